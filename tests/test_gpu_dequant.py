@@ -54,6 +54,16 @@ def test_crafted_blocks_bit_exact(device, orc, qtype, mode):
     compare(dequant(device, qtype, data, n, mode), orc.dequantize(qtype, data, n, mode))
 
 
+@pytest.mark.parametrize("elems", [256, 1792, 2048, 2304, 4096, 6400, 8448])
+@pytest.mark.parametrize("qtype", TYPES)
+def test_workgroup_edges_bit_exact(device, orc, qtype, elems):
+    # a workgroup step covers 2048 outputs (Q6_K 4096): less than one, whole ones, a rest
+    data = crafted_blocks(qtype, elems // QK[qtype], seed=elems + qtype)
+    for n in {elems, elems - QK[qtype]} - {0}:
+        part = data[:n // QK[qtype] * BB[qtype]]
+        compare(dequant(device, qtype, part, n, nat.F16_IEEE), orc.dequantize(qtype, part, n, nat.F16_IEEE))
+
+
 @pytest.mark.parametrize("mode", [nat.F16_IEEE, nat.F16_REFCPU])
 @pytest.mark.parametrize("qtype,n,k", [(nat.Q4_K, 14336, 4096), (nat.Q6_K, 4096, 14336),
                                        (nat.Q8_0, 4096, 4096), (nat.Q4_0, 14336, 4096)])
