@@ -158,12 +158,14 @@ struct aih_rope_qkv_args {
     int32_t start = 0, qd = 0, kvd = 0, head_dim = 0, table_rows = 0;
 };
 
-// may_split: the GEMM may split K over workgroups, with partial sums in the
-// second workspace and a reduction (never with caller-provided staging).
-// rope: the epilogue's arguments for epi 3 (else unused).
+// may_split: a GEMM of more than 256 rows may split K over workgroups, with
+// partial sums in the second workspace and a summing pass (never with
+// caller-provided staging); one of at most 256 rows splits by its shape alone.
+// rope: the epilogue's arguments for epi 3 (else unused).  room: memory for
+// partial sums, 16-byte aligned, in place of the second workspace.
 int aih_launch_qgemm_tiled(aih_ctx *ctx, int type, const void *W, int64_t N, int64_t K, const void *Xt,
                            int64_t M, float *Y, int epi, bool may_split = false,
-                           const aih_rope_qkv_args *rope = nullptr);
+                           const aih_rope_qkv_args *rope = nullptr, const aih_scratch *room = nullptr);
 int aih_launch_qmatvec_mfma(aih_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
                             const float *X, int64_t ldx, float *Y, int64_t ldy, int batch,
                             const aih_scratch *ext = nullptr);

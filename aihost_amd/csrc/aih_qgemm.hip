@@ -14,14 +14,14 @@
 // conversion is aih_decoder.hip's x_tile_pre_kernel, which also computes the
 // element-wise step before the GEMM when there is one).  A
 // workgroup then owns a 128 (M) x 64 (N) tile of Y and walks K in super-steps
-// of 256 elements: four producer waves dequantize W for the next super-step
+// of 256 elements: producer waves dequantize W for the next super-step
 // into LDS while four consumer waves multiply the current one, their A
 // fragments loaded straight from the tiled X (see qgemm_kernel).  Large grids
 // use 256 x 64 or 512 x 64 tiles with every wave in both roles
-// (qgemm256_kernel); tall products whose 512-row grid leaves CUs idle split
-// K over workgroups and sum the partials in a second pass
-// (split_k_sum_kernel).  The epilogue stores Y or adds into it (the residual
-// add of a layer).
+// (qgemm256_kernel); products whose grid leaves CUs idle split K over
+// workgroups and sum the partials in a second pass (plan_gemm,
+// launch_split_sum).  The epilogue stores Y or adds into it (the residual add
+// of a layer), or is one of the fused ones below.
 //
 // Precision.  Both operands are rounded to fp16 (11-bit significand) and the
 // products accumulate in fp32: normwise error near 3e-4 against the fp32
@@ -261,33 +261,37 @@ __device__ __forceinline__ void rope_qkv_tile(const f16v &acc0, const f16v &acc1
     rope_qkv_block(acc1, lane, mrow0, n0 + 32, M, N, Y, ra);
 }
 
-// Eight waves per workgroup in two roles, one of each on every SIMD; the
-// workgroup owns a 128 (M) x 64 (N) tile of Y and walks K in super-steps of
-// 256 (a Q4_K/Q6_K super-block, 8 blocks of Q8_0/Q4_0), with one LDS barrier
-// per super-step and two tile buffers.
-//   Producers (waves 4..7) dequantize the next super-step of the 64 weight
-//   rows into LDS: wave p owns rows 16p .. 16p+15.  For Q4_K, Q4_0 and Q8_0
+// Waves in two roles: eight producers (four for Q8_0) and four consumers, one
+// consumer per SIMD; the workgroup owns a 128 (M) x 64 (N) tile of Y and walks
+// K in super-steps of 256 (a Q4_K/Q6_K super-block, 8 blocks of Q8_0/Q4_0),
+// with one LDS barrier per super-step and two tile buffers.
+//   Producers (waves 4..) dequantize the next super-step of the 64 weight
+//   rows into LDS: each owns RPW consecutive rows.  For Q4_K, Q4_0 and Q8_0
 //   eight lanes per row take 32 weights each (the wide-tile kernel's pieces
-//   and LDS positions: two row groups of 8 per wave); for Q6_K sixteen lanes
-//   per row take pieces 0..15 of the row's 256-k span (four row groups of 4,
-//   each row read as one contiguous span), which measured faster there
-//   (4096 x 4096 x 512: 39.9 against 40.5 us per call; the 32-weight form
-//   gave Q4_0 36.2 -> 34.6 and Q8_0 36.5 -> 35.9).  Their packed loads run
-//   PR super-steps ahead in a ring of register sets.
+//   and LDS positions); for Q6_K sixteen lanes per row take pieces 0..15 of
+//   the row's 256-k span (each row read as one contiguous span), which
+//   measured faster there.  Their packed loads run PR super-steps ahead in a
+//   ring of register sets.  A single producer wave per SIMD issues its
+//   dependent conversions at 5 to 7 cycles each; two fill each other's gaps
+//   (4096 x 4096 x 512 per call, four against eight producers: Q4_K 35.1 ->
+//   33.0 us, Q4_0 33.4 -> 32.3, Q6_K 39.5 -> 38.4; 4096 x 14336 x 33 unsplit,
+//   Q4_K 69.3 -> 59.4).  Q8_0, bound by its 34-byte blocks' unaligned loads,
+//   gained nothing there and lost 1-3% where its weights fill the memory
+//   (32000 x 14336 x 64: 198 against 203 us): it keeps four.
 //   Consumers (waves 0..3): wave w owns rows 32w .. 32w+31 of the M tile and
 //   all 64 columns (two 32x32 accumulators sharing each A fragment).  A
 //   fragments come straight from the tiled fp16 copy of X, one super-step
 //   ahead; B fragments from LDS.
-// On MI355X the 4096 x 4096 x 512 Q4_K product takes 35-37 us per call (the
-// kernel 27-28 us, the X conversion 7.5 us), against 42 us for an earlier
-// form with one barrier per 64 k.
+// On MI355X the 4096 x 4096 x 512 Q4_K product takes 33 us per call (the
+// kernel about 25 us, the X conversion 7.5 us).
 constexpr int SK = 256;            // k per super-step (one barrier)
 constexpr int SC = SK / 64;        // 64-k steps per super-step
 constexpr int LD2 = SK + 8;        // LDS row stride in halves (16-byte pad against bank conflicts)
-// producer ring depth in super-steps (Q6_K's larger raw sets: 2, within 256
-// registers) and piece layout (P32: 32-weight pieces, else 16-weight)
-template <class T> struct GRing { static constexpr int PR = 3; static constexpr bool P32 = true; };
-template <> struct GRing<G6K> { static constexpr int PR = 2; static constexpr bool P32 = false; };
+// producer waves, their ring depth in super-steps (Q6_K's larger raw sets: 2)
+// and piece layout (P32: 32-weight pieces, else 16-weight)
+template <class T> struct GRing { static constexpr int NP = 8, PR = 3; static constexpr bool P32 = true; };
+template <> struct GRing<G6K> { static constexpr int NP = 8, PR = 2; static constexpr bool P32 = false; };
+template <> struct GRing<G80> { static constexpr int NP = 4, PR = 3; static constexpr bool P32 = true; };
 
 // LDS position (in 16-byte granules) of chunk granule g of a super-step (the
 // k values 8g .. 8g+7): the 32-weight pieces' swizzle, or for 16-weight
@@ -301,35 +305,40 @@ template <class T> struct BPos<T, false> {
 };
 
 template <class T>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(64 * (4 + GRing<T>::NP))
 qgemm_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
-             const _Float16 *__restrict__ Xt, int64_t M, float *__restrict__ Y, int epi, aih_rope_qkv_args ra)
+             const _Float16 *__restrict__ Xt, int64_t M, float *__restrict__ Y, int epi, float *__restrict__ P,
+             int64_t zs, int ssper, aih_rope_qkv_args ra)
 {
     constexpr int PR = GRing<T>::PR;
     constexpr bool P32 = GRing<T>::P32;
     typedef typename Piece32<T>::type Pc;
     typedef std::conditional_t<P32, typename Pc::Raw, typename T::Raw> Raw;
-    constexpr int NR = P32 ? 2 : 4;   // row groups per producer wave
+    constexpr int RPW = BN / GRing<T>::NP;   // weight rows per producer wave
+    constexpr int NR = P32 ? RPW / 8 : RPW / 4;   // row groups per producer wave
     __shared__ __align__(16) _Float16 wsh[2][BN][LD2];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
     const int nch = (int)(K / 64);
-    const int nss = (nch + SC - 1) / SC;
+    // split z of K (gridDim.z > 1: partial sums into P + z * zs): super-steps
+    // ss0 .. ss0 + nss - 1; chunk indices below stay absolute
+    const int ss0 = (int)blockIdx.z * ssper;
+    const int nss = min(ssper, (nch + SC - 1) / SC - ss0);
 
     if (wave >= 4) {
-        // rows 16 pw + (16 / NR) i + rl; P32: chunk pc, half ps of it (32
+        // rows RPW pw + (RPW / NR) i + rl; P32: chunk pc, half ps of it (32
         // weights); else chunk pc, piece ps (16 weights)
         const int pw = wave - 4;
-        constexpr int LPR = 64 * NR / 16;   // lanes per row
+        constexpr int LPR = 64 * NR / RPW;   // lanes per row
         const int rl = lane / LPR, p = lane % LPR, pc = p / (LPR / 4), ps = p % (LPR / 4);
         const uint8_t *wrow[NR];
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
-            const int64_t wn = n0 + 16 * pw + (16 / NR) * i + rl;
+            const int64_t wn = n0 + RPW * pw + (RPW / NR) * i + rl;
             wrow[i] = W + (wn < N ? wn : N - 1) * row_bytes;
         }
         auto gload = [&](int ss, Raw *r) {
-            int c = ss * SC + pc;
+            int c = (ss0 + ss) * SC + pc;
             c = c < nch ? c : nch - 1;
 #pragma unroll
             for (int i = 0; i < NR; ++i) {
@@ -341,11 +350,11 @@ qgemm_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
         // zeros: only the stages after the main loop test for them
         auto stage = [&](auto tail, int ss, int buf, const Raw *r) {
             asm volatile("" : "+s"(ss));
-            const int c = ss * SC + pc;
+            const int c = (ss0 + ss) * SC + pc;
             const bool zero = decltype(tail)::value && c >= nch;
 #pragma unroll
             for (int i = 0; i < NR; ++i) {
-                _Float16 *d = &wsh[buf][16 * pw + (16 / NR) * i + rl][0];
+                _Float16 *d = &wsh[buf][RPW * pw + (RPW / NR) * i + rl][0];
                 if constexpr (P32) {
                     h8 o[4];
                     Pc::piece(r[i], c, ps, o);
@@ -403,6 +412,7 @@ qgemm_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
     const int32_t ev = E[mb * 32 + (lane & 31)];
     struct AF { h8 a[4]; };
     auto aload = [&](int kb, AF &f) {
+        kb += SC * ss0;
         kb = kb < nch ? kb : nch - 1;
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) f.a[kk] = ldg<h8>(xa + ((int64_t)kb * 4 + kk) * 512);
@@ -451,12 +461,16 @@ qgemm_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
         bload(buf, 0, bb[0]);
 #pragma unroll
         for (int t = 0; t < SC; ++t) {
-            if (t + 1 < SC && SC * ss + t + 1 < nch) bload(buf, t + 1, bb[(t + 1) & 1]);
-            if (SC * ss + t < nch) mm(f[t], bb[t & 1]);
+            if (t + 1 < SC && SC * (ss0 + ss) + t + 1 < nch) bload(buf, t + 1, bb[(t + 1) & 1]);
+            if (SC * (ss0 + ss) + t < nch) mm(f[t], bb[t & 1]);
         }
     }
 
     undo_row_exp(acc0, acc1, ev, E, mb * 32, lane);
+    if (P) {   // a split's partial sums (the summing pass applies the epilogue)
+        store_tile(acc0, acc1, lane, m0 + 32 * wave, n0, M, N, P + (int64_t)blockIdx.z * zs, false);
+        return;
+    }
     if (epi == kEpiSiluOperand) {
         // the tile buffer of super-step nss: nothing reads or writes it any more
         silu_pairs_operand(acc0, acc1, lane, m0 + 32 * wave, n0, M, N,
@@ -493,7 +507,7 @@ template <class T, int MB, int AD>
 __global__ void __launch_bounds__(512)
 qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
                 const _Float16 *__restrict__ Xt, int64_t M, float *__restrict__ Y, int epi,
-                float *__restrict__ P, int ssper, aih_rope_qkv_args ra)
+                float *__restrict__ P, int64_t zs, int ssper, aih_rope_qkv_args ra)
 {
     static_assert(SC % AD == 0, "A ring depth divides a super-step");
     constexpr int PR = PR256;
@@ -503,7 +517,7 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t m0 = (int64_t)blockIdx.y * BM2 * MB, n0 = (int64_t)blockIdx.x * BN;
     const int nch = (int)(K / 64);
-    // split z of K (gridDim.z > 1: partial sums into P): super-steps
+    // split z of K (gridDim.z > 1: partial sums into P + z * zs): super-steps
     // ss0 .. ss0 + nss - 1; chunk indices below stay absolute
     const int ss0 = (int)blockIdx.z * ssper;
     const int nss = min(ssper, (nch + SC - 1) / SC - ss0);
@@ -653,38 +667,119 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
         }
         return;
     }
-    if (epi == kEpiRopeQKV) {   // never split (the plan does not split this epilogue)
+    if (epi == kEpiRopeQKV) {   // never split here (the plan splits this epilogue over 128-row tiles only)
 #pragma unroll
         for (int j = 0; j < MB; ++j) rope_qkv_tile(acc[j][0], acc[j][1], lane, m0 + 32 * (MB * wave + j), n0, M, N, Y, ra);
         return;
     }
     // a split's partial sums are stored (the summing pass adds them into Y)
-    float *const Pz = P ? P + (int64_t)blockIdx.z * M * N : nullptr;
+    float *const Pz = P ? P + (int64_t)blockIdx.z * zs : nullptr;
 #pragma unroll
     for (int j = 0; j < MB; ++j)
         store_tile(acc[j][0], acc[j][1], lane, m0 + 32 * (MB * wave + j), n0, M, N, Pz ? Pz : Y,
                    !Pz && epi == kEpiAccumulate);
 }
 
+// The sum of the splits' partial sums p[0], p[zs], ... (in that order).
+__device__ __forceinline__ f4 split_sum4(const float *__restrict__ p, int S, int64_t zs)
+{
+    f4 s = *reinterpret_cast<const f4 *>(p);
+    int z = 1;
+    for (; z + 4 <= S; z += 4) {   // four splits' loads in flight
+        f4 v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const f4 *>(p + (int64_t)(z + j) * zs);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s += v[j];
+    }
+    for (; z < S; ++z) s += *reinterpret_cast<const f4 *>(p + (int64_t)z * zs);
+    return s;
+}
+
 // The splits of a GEMM split over K: Y = P_0 + P_1 + ... (in that order),
 // added into Y (Y + sum, the order of the accumulate epilogue) when
-// `accumulate`.  Four elements per thread (16-byte accesses of Y when it is
-// 16-byte aligned).
+// `accumulate`.  Splits are zs floats apart (a multiple of 4, at least MN).
+// Four elements per thread (16-byte accesses of Y when it is 16-byte aligned).
 template <bool VEC>
 __global__ void __launch_bounds__(256)
-split_k_sum_kernel(const float *__restrict__ P, int S, int64_t MN, float *__restrict__ Y, int accumulate)
+split_k_sum_kernel(const float *__restrict__ P, int S, int64_t MN, int64_t zs, float *__restrict__ Y, int accumulate)
 {
     for (int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x); i < MN; i += 4 * (int64_t)gridDim.x * 256) {
-        f4 s = *reinterpret_cast<const f4 *>(P + i);
-        for (int z = 1; z < S; ++z) s += *reinterpret_cast<const f4 *>(P + (int64_t)z * MN + i);
-        if (VEC) {
+        const f4 s = split_sum4(P + i, S, zs);
+        if (VEC && i + 4 <= MN) {
             f4 *y = reinterpret_cast<f4 *>(Y + i);
             *y = accumulate ? *y + s : s;
         } else {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) Y[i + j] = accumulate ? Y[i + j] + s[j] : s[j];
+            for (int j = 0; j < 4; ++j)
+                if (i + j < MN) Y[i + j] = accumulate ? Y[i + j] + s[j] : s[j];
         }
     }
+}
+
+// The same sum with the Q|K|V epilogue: what rope_qkv_block stores, two pairs
+// (four columns) per thread.  N and the head boundaries are multiples of 32.
+__global__ void __launch_bounds__(256)
+split_k_rope_kernel(const float *__restrict__ P, int S, int64_t M, int64_t N, int64_t zs, float *__restrict__ Y,
+                    const aih_rope_qkv_args ra)
+{
+#pragma clang fp contract(off)
+    const int64_t t = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
+    if (t >= M * N) return;
+    const int64_t m = t / N, n = t % N;
+    const f4 x = split_sum4(P + t, S, zs);
+    const int64_t p = (int64_t)ra.start + (ra.pos ? *ra.pos : 0) + m;
+    const bool in_table = p >= 0 && p < ra.table_rows, in_cache = in_table && p < ra.cache_rows;
+    const int kind = n < ra.qd ? 0 : n < (int64_t)ra.qd + ra.kvd ? 1 : 2;
+    f4 v = x;
+    if (kind < 2 && in_table) {
+        const int64_t cn = kind == 0 ? n : n - ra.qd;
+        const float *c = ra.table + 2 * (p * (ra.head_dim / 2) + cn % ra.head_dim / 2);
+        v = f4{x.x * c[0] - x.y * c[1], x.x * c[1] + x.y * c[0], x.z * c[2] - x.w * c[3], x.z * c[3] + x.w * c[2]};
+    }
+    float *to;
+    if (kind == 0) to = Y + t;
+    else if (!in_cache) return;
+    else if (kind == 1) to = ra.Kc + p * ra.kvd + (n - ra.qd);
+    else to = ra.Vc + p * ra.kvd + (n - ra.qd - ra.kvd);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) to[j] = v[j];
+}
+
+// The same sum with the SiLU-pairs operand epilogue: what silu_pairs_operand
+// writes.  Thread t of a row holds 16 columns (8 outputs, one 16-byte slot of
+// the image); the four threads of a 32-output block share its exponent.
+// N is a multiple of 64; rows M .. mpad - 1 are zero.
+__global__ void __launch_bounds__(256)
+split_k_silu_kernel(const float *__restrict__ P, int S, int64_t M, int64_t N, int64_t zs, _Float16 *__restrict__ out)
+{
+    const int64_t mpad = aih_operand::mpad_of(M), kd = N / 2, per_row = N / 16;
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t m = t / per_row, c = t % per_row;
+    const bool live = m < M;   // whole groups of four threads alike (per_row is a multiple of 4)
+    float v[8] = {};
+    if (live) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f4 x = split_sum4(P + m * N + 16 * c + 4 * q, S, zs);
+            v[2 * q] = (x.x * (1.0f / (1.0f + expf(-x.x)))) * x.y;
+            v[2 * q + 1] = (x.z * (1.0f / (1.0f + expf(-x.z)))) * x.w;
+        }
+    }
+    float mx = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fabsf(v[j]));
+    mx = fmaxf(mx, __shfl_xor(mx, 1));
+    mx = fmaxf(mx, __shfl_xor(mx, 2));
+    if (m >= mpad) return;
+    const int eb = aih_operand::block_exp(mx), e = eb == aih_operand::kZeroBlock ? 0 : eb;
+    h8 h;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) h[j] = (_Float16)ldexpf(v[j], e);
+    *reinterpret_cast<h8 *>(out + aih_operand::slot_half(m, 8 * c, kd)) = h;
+    char *const img = reinterpret_cast<char *>(out);
+    if (c % 4 == 0) reinterpret_cast<int8_t *>(img + aih_operand::block_exp_offset(mpad, kd))[m * (kd / 32) + c / 4] = (int8_t)eb;
+    if (c == 0) reinterpret_cast<int32_t *>(img + aih_operand::row_exp_offset(mpad, kd))[m] = 0;
 }
 
 // Before a GEMM reads an image written one 32-column block at a time
@@ -742,8 +837,8 @@ operand_fixup_kernel(_Float16 *__restrict__ Xt, int64_t mpad, int64_t K)
 }
 
 // The tiling of a GEMM: rows per workgroup tile (128, 256 or 512) and, for
-// 512-row tiles, the number of K splits (splits > 1: partial sums in the
-// second workspace, then split_k_sum_kernel) of ssper super-steps each.
+// 128- and 512-row tiles, the number of K splits (splits > 1: partial sums in
+// the second workspace, then a summing pass) of ssper super-steps each.
 struct GemmPlan {
     int tile = 128;
     int splits = 1;
@@ -761,6 +856,20 @@ struct GemmPlan {
 // output, plus 2 us of launch; a 128-row workgroup takes about 29 us per
 // 4096 of K).  The plan depends only on the shape, the epilogue, the CU count
 // and whether the call may split, never on what the context has allocated.
+//
+// Products of at most 256 rows split the 128-row tiles over K, at most 8 ways,
+// when those leave CUs idle (a 4096-row weight has 64 tiles).  A workgroup
+// takes about 3 us and 1.1 us per super-step, and the summing pass 4 us and
+// its traffic at 2.5 TB/s.  Every entry point and epilogue splits a shape
+// alike, so the operand image and the partial sums together stay within the
+// allocation-free entry point's buffer.
+// Measured per call (Q4_K / Q6_K, whole -> split): 4096 x 14336 x 33 69 -> 28
+// / 82 -> 32 us, 4096 x 4096 x 33 24 -> 15 / 28 -> 17, x 256 27 -> 24 / 31 ->
+// 26, 1024 x 14336 x 64 71 -> 21 / 84 -> 23, 8192 x 4096 x 9 25 -> 18 / 30 ->
+// 21; over 216 sizes of N 1024-32000, K 1024-14336 and M 9-256 none slower
+// than the runs differ.
+int64_t split_stride(int64_t M, int64_t N) { return (M * N + 3) / 4 * 4; }
+
 GemmPlan plan_gemm(int64_t cu_count, int64_t N, int64_t K, int64_t M, int epi, bool may_split)
 {
     const int64_t gx = (N + BN - 1) / BN, gy = (M + BM - 1) / BM, gy2 = (M + BM2 - 1) / BM2;
@@ -771,6 +880,25 @@ GemmPlan plan_gemm(int64_t cu_count, int64_t N, int64_t K, int64_t M, int epi, b
     const int nss = (int)((K / 64 + SC - 1) / SC);
     GemmPlan p;
     p.ssper = nss;
+    if (M <= BM2) {
+        const size_t image = (size_t)aih_operand::image_bytes(aih_operand::mpad_of(M), K, false);
+        const size_t room = image < AIH_NOALLOC_SCRATCH_BYTES ? AIH_NOALLOC_SCRATCH_BYTES - image : 0;
+        const double whole = 3.0 + 1.1 * nss;
+        double best = std::min(c1, c2) / 20.0 * whole;
+        for (int want = 2; want <= 8 && 2 * want <= nss; ++want) {
+            const int ssper = (nss + want - 1) / want;
+            const int S = (nss + ssper - 1) / ssper;
+            const size_t bytes = (size_t)S * (size_t)split_stride(M, N) * sizeof(float);
+            if (bytes > room) break;
+            const double us = rounds(gx * gy * S) * (3.0 + 1.1 * ssper) + 4.0 + (double)bytes / 2.5e6;
+            if (us < best) {
+                best = us;
+                p.splits = S;
+                p.ssper = ssper;
+            }
+        }
+        if (p.splits > 1) return p;
+    }
     if (may_split && epi != kEpiSiluOperand && epi != kEpiRopeQKV && M > BM2 && gx * gy4 < cus && M * N % 4 == 0) {
         const int want = (int)std::min<int64_t>(std::min<int64_t>(cus / (gx * gy4), nss / 2), 8);
         if (want >= 2) {
@@ -791,53 +919,81 @@ GemmPlan plan_gemm(int64_t cu_count, int64_t N, int64_t K, int64_t M, int epi, b
     return p;
 }
 
+// The summing pass of a split product, with its epilogue.
+int launch_split_sum(aih_ctx *ctx, const float *P, const GemmPlan &p, int64_t M, int64_t N, float *Y, int epi,
+                     const aih_rope_qkv_args &ra)
+{
+    const int64_t zs = split_stride(M, N);
+    if (epi == kEpiRopeQKV) {
+        hipLaunchKernelGGL(split_k_rope_kernel, dim3((unsigned)((M * N / 4 + 255) / 256)), dim3(256), 0, ctx->stream, P,
+                           p.splits, M, N, zs, Y, ra);
+        return aih_launch_status();
+    }
+    if (epi == kEpiSiluOperand) {
+        const int64_t threads = aih_operand::mpad_of(M) * (N / 16);
+        hipLaunchKernelGGL(split_k_silu_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, ctx->stream, P,
+                           p.splits, M, N, zs, reinterpret_cast<_Float16 *>(Y));
+        return aih_launch_status();
+    }
+    const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    const int64_t groups = ((M * N + 3) / 4 + 255) / 256;
+    const dim3 grid((unsigned)std::min<int64_t>(groups, 8 * cus));
+    const int add = epi == kEpiAccumulate ? 1 : 0;
+    if (reinterpret_cast<uintptr_t>(Y) % 16 == 0)
+        hipLaunchKernelGGL(split_k_sum_kernel<true>, grid, dim3(256), 0, ctx->stream, P, p.splits, M * N, zs, Y, add);
+    else
+        hipLaunchKernelGGL(split_k_sum_kernel<false>, grid, dim3(256), 0, ctx->stream, P, p.splits, M * N, zs, Y, add);
+    return aih_launch_status();
+}
+
+// room: staging memory for partial sums that the caller supplies (the
+// allocation-free entry point), else the second workspace.
 template <class T>
-int launch(aih_ctx *ctx, const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
-           const _Float16 *Xh, int64_t M, float *Y, int epi, bool may_split, const aih_rope_qkv_args &ra)
+int launch(aih_ctx *ctx, const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes, const _Float16 *Xh, int64_t M,
+           float *Y, int epi, bool may_split, const aih_rope_qkv_args &ra, const aih_scratch *room)
 {
     const int64_t gx = (N + BN - 1) / BN, gy = (M + BM - 1) / BM, gy2 = (M + BM2 - 1) / BM2;
     const int64_t gy4 = (M + 2 * BM2 - 1) / (2 * BM2);
     if (gy > 65535 || gx > 0x7FFFFFFF) return AIH_E_LIMIT;
-    const GemmPlan p = plan_gemm(ctx->cu_count, N, K, M, epi, may_split);
+    GemmPlan p = plan_gemm(ctx->cu_count, N, K, M, epi, may_split);
+    const int64_t zs = split_stride(M, N);
+    void *ws = nullptr;
     if (p.splits > 1) {
-        // the split's partial sums: a shape that splits always splits (a
-        // workspace that cannot grow here, as during a graph capture, is an
-        // error, not a silent change of summation order)
-        void *ws = nullptr;
-        int rc = aih_workspace2(ctx, (size_t)p.splits * (size_t)(M * N) * sizeof(float), &ws);
-        if (rc) return rc;
-        hipLaunchKernelGGL((qgemm256_kernel<T, 2, 2>), dim3((unsigned)gx, (unsigned)gy4, (unsigned)p.splits),
-                           dim3(512), 0, ctx->stream, W, N, K, row_bytes, Xh, M, Y, epi, static_cast<float *>(ws),
-                           p.ssper, ra);
-        rc = aih_launch_status();
-        if (rc) return rc;
-        const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-        const int64_t groups = (M * N / 4 + 255) / 256;
-        const dim3 grid((unsigned)std::min<int64_t>(groups, 8 * cus));
-        if (reinterpret_cast<uintptr_t>(Y) % 16 == 0)
-            hipLaunchKernelGGL(split_k_sum_kernel<true>, grid, dim3(256), 0, ctx->stream,
-                               static_cast<const float *>(ws), p.splits, M * N, Y, epi == kEpiAccumulate ? 1 : 0);
-        else
-            hipLaunchKernelGGL(split_k_sum_kernel<false>, grid, dim3(256), 0, ctx->stream,
-                               static_cast<const float *>(ws), p.splits, M * N, Y, epi == kEpiAccumulate ? 1 : 0);
-        return aih_launch_status();
+        const size_t bytes = (size_t)p.splits * (size_t)zs * sizeof(float);
+        int rc = AIH_OK;
+        if (room && bytes <= room->bytes) ws = room->ptr;
+        else rc = room ? AIH_E_SCRATCH : aih_workspace2(ctx, bytes, &ws);
+        if (rc) {
+            // 512-row tiles: a shape that splits always splits (a workspace
+            // that cannot grow here, as during a graph capture, is an error).
+            // 128-row tiles: their partial sums fit the workspace that
+            // aih_init sets aside; without it the product runs whole.
+            if (p.tile != BM) return rc;
+            ws = nullptr;
+            p.splits = 1;
+            p.ssper = (int)((K / 64 + SC - 1) / SC);
+        }
     }
+    float *const P = static_cast<float *>(ws);
+    const unsigned gz = (unsigned)p.splits;
     if (p.tile == 512)
-        hipLaunchKernelGGL((qgemm256_kernel<T, 2, 2>), dim3((unsigned)gx, (unsigned)gy4), dim3(512), 0, ctx->stream,
-                           W, N, K, row_bytes, Xh, M, Y, epi, nullptr, p.ssper, ra);
+        hipLaunchKernelGGL((qgemm256_kernel<T, 2, 2>), dim3((unsigned)gx, (unsigned)gy4, gz), dim3(512), 0, ctx->stream,
+                           W, N, K, row_bytes, Xh, M, Y, epi, P, zs, p.ssper, ra);
     else if (p.tile == 256)
         hipLaunchKernelGGL((qgemm256_kernel<T, 1, SC>), dim3((unsigned)gx, (unsigned)gy2), dim3(512), 0, ctx->stream,
-                           W, N, K, row_bytes, Xh, M, Y, epi, nullptr, p.ssper, ra);
+                           W, N, K, row_bytes, Xh, M, Y, epi, P, zs, p.ssper, ra);
     else
-        hipLaunchKernelGGL((qgemm_kernel<T>), dim3((unsigned)gx, (unsigned)gy), dim3(512), 0, ctx->stream,
-                           W, N, K, row_bytes, Xh, M, Y, epi, ra);
-    return aih_launch_status();
+        hipLaunchKernelGGL((qgemm_kernel<T>), dim3((unsigned)gx, (unsigned)gy, gz), dim3(64 * (4 + GRing<T>::NP)), 0, ctx->stream,
+                           W, N, K, row_bytes, Xh, M, Y, epi, P, zs, p.ssper, ra);
+    const int rc = aih_launch_status();
+    return rc || p.splits == 1 ? rc : launch_split_sum(ctx, P, p, M, N, Y, epi, ra);
 }
 
 }  // namespace
 
 int aih_launch_qgemm_tiled(aih_ctx *ctx, int type, const void *W, int64_t N, int64_t K, const void *Xtv,
-                           int64_t M, float *Y, int epi, bool may_split, const aih_rope_qkv_args *rope)
+                           int64_t M, float *Y, int epi, bool may_split, const aih_rope_qkv_args *rope,
+                           const aih_scratch *room)
 {
     const aih_rope_qkv_args ra = rope ? *rope : aih_rope_qkv_args{};
     if (K % BK != 0) return AIH_E_LIMIT;
@@ -845,10 +1001,10 @@ int aih_launch_qgemm_tiled(aih_ctx *ctx, int type, const void *W, int64_t N, int
     const uint8_t *w = static_cast<const uint8_t *>(W);
     const _Float16 *Xt = static_cast<const _Float16 *>(Xtv);
     switch (type) {
-    case AIH_TYPE_Q4_K: return launch<G4K>(ctx, w, N, K, rb, Xt, M, Y, epi, may_split, ra);
-    case AIH_TYPE_Q6_K: return launch<G6K>(ctx, w, N, K, rb, Xt, M, Y, epi, may_split, ra);
-    case AIH_TYPE_Q8_0: return launch<G80>(ctx, w, N, K, rb, Xt, M, Y, epi, may_split, ra);
-    case AIH_TYPE_Q4_0: return launch<G40>(ctx, w, N, K, rb, Xt, M, Y, epi, may_split, ra);
+    case AIH_TYPE_Q4_K: return launch<G4K>(ctx, w, N, K, rb, Xt, M, Y, epi, may_split, ra, room);
+    case AIH_TYPE_Q6_K: return launch<G6K>(ctx, w, N, K, rb, Xt, M, Y, epi, may_split, ra, room);
+    case AIH_TYPE_Q8_0: return launch<G80>(ctx, w, N, K, rb, Xt, M, Y, epi, may_split, ra, room);
+    case AIH_TYPE_Q4_0: return launch<G40>(ctx, w, N, K, rb, Xt, M, Y, epi, may_split, ra, room);
     default: return AIH_E_UNSUPPORTED;
     }
 }
@@ -877,7 +1033,13 @@ int aih_launch_qgemm(aih_ctx *ctx, int type, const void *W, int64_t N, int64_t K
     if (rc) return rc;
     rc = aih_launch_x_tile(ctx, X, M, K, work);
     if (rc) return rc;
-    return aih_launch_qgemm_tiled(ctx, type, W, N, K, work, M, Y, 0, may_split && ext == nullptr);
+    aih_scratch room = {};
+    if (ext) {
+        const size_t image = (size_t)aih_operand::image_bytes(aih_operand::mpad_of(M), K, false);   // a multiple of 128
+        room = {static_cast<char *>(work) + image, ext->bytes - image};
+    }
+    return aih_launch_qgemm_tiled(ctx, type, W, N, K, work, M, Y, 0, may_split && ext == nullptr, nullptr,
+                                  ext ? &room : nullptr);
 }
 
 extern "C" int aih_qgemm_plan(aih_ctx *ctx, int64_t N, int64_t K, int64_t M, int may_split, int32_t *tile_rows,

@@ -227,6 +227,10 @@ int aih_init(int device_index, aih_ctx **out)
         release(ctx);
         return (int)err;
     }
+    // room for the partial sums of GEMMs of at most 256 rows (plan_gemm), so
+    // that they split alike inside a graph capture; without it they run whole
+    void *reserved = nullptr;
+    (void)aih_workspace2(ctx, AIH_NOALLOC_SCRATCH_BYTES, &reserved);
     *out = ctx;
     return AIH_OK;
 }
@@ -598,8 +602,9 @@ int matmul_weights_q(aih_ctx *ctx, int type, const void *W, int64_t N, int64_t K
                      float *Y, const aih_scratch *ext)
 {
     if (M >= 1 && M <= 8) return qmatvec(ctx, type, W, N, K, X, K, Y, N, (int)M, ext);
-    // never split over K: the allocation-free variant, which shares this
-    // path, has no room for partial sums, and both return the same bits
+    // more than 256 rows never split over K: the allocation-free variant,
+    // which shares this path, has no room for their partial sums, and both
+    // return the same bits
     return qgemm(ctx, type, W, N, K, X, M, Y, ext, false);
 }
 

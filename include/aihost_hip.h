@@ -254,8 +254,10 @@ int aih_qmatvec_fused(aih_ctx *ctx, int type, const void *W, int64_t N, int64_t 
  * to a second context workspace under the same rules and are added in a
  * fixed order, so a result depends only on the shape (and the device's CU
  * count), not on the call; where that workspace cannot grow (during a
- * capture, out of memory), the call fails like the X workspace's.  Replaces
- * TempF32 + ComputeOps.MatMulWeights for M > 8. */
+ * capture, out of memory), the call fails like the X workspace's.  One of at
+ * most 256 rows does so too, in every entry point and with every epilogue
+ * alike, with partial sums that fit a workspace set aside by aih_init.
+ * Replaces TempF32 + ComputeOps.MatMulWeights for M > 8. */
 int aih_qgemm(aih_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
               const float *X, int64_t M, float *Y);
 
@@ -270,8 +272,9 @@ int aih_qgemm_plan(aih_ctx *ctx, int64_t N, int64_t K, int64_t M, int may_split,
                    int32_t *splits);
 
 /* ComputeOps.MatMulWeights semantics for a quantized weight: routes M <= 8 to
- * aih_qmatvec and larger M to aih_qgemm, never split over K (the results of
- * aih_matmul_weights_q_noalloc, which has no room for partial sums). */
+ * aih_qmatvec and larger M to aih_qgemm; more than 256 rows are never split
+ * over K (the results of aih_matmul_weights_q_noalloc, which has no room for
+ * their partial sums). */
 int aih_matmul_weights_q(aih_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
                          const float *X, int64_t M, float *Y);
 

@@ -97,6 +97,41 @@ def test_split_k(device, orc, qtype, n, k, m):
     assert np.linalg.norm(y - ref) / np.linalg.norm(ref) < 1e-6
 
 
+# Products of at most 256 rows whose 128-row tiles leave CUs idle split K in
+# every entry point: row and column remainders (M x N odd: the last outputs
+# are stored one by one, as are all when Y is not 16-byte aligned), 64-k
+# remainders inside the last split, two row tiles.  The oracle's bound, and
+# the same bits from the allocation-free entry point.
+@pytest.mark.parametrize("qtype,n,k,m,offset", [
+    (nat.Q4_K, 1024, 14336, 33, 0), (nat.Q6_K, 1001, 4096, 9, 0), (nat.Q6_K, 63, 2048, 127, 4),
+    (nat.Q8_0, 517, 4160, 129, 0), (nat.Q4_0, 999, 3136, 255, 12), (nat.Q4_0, 1, 2048, 9, 0),
+    (nat.Q4_K, 4096, 4096, 256, 0),
+])
+def test_small_grid_split_k(device, orc, qtype, n, k, m, offset):
+    tile, splits = nat.qgemm_plan(device.handle, n, k, m)
+    assert nat.qgemm_plan(device.handle, n, k, m, may_split=False) == (tile, splits)
+    if device.info().compute_units == 256 and (n, k, m) != (4096, 4096, 256):
+        assert (tile, splits > 1) == (128, True)
+    w = synth_weight(qtype, n, k, seed=n + k + 2)
+    x = x_of(m, k, seed=m + 6)
+    wb, xb, yb = upload(device, w), upload(device, x), device.create_buffer(m * n * 4 + 32)
+    try:
+        got = []
+        for fn in (nat.lib().aih_matmul_weights_q, nat.lib().aih_matmul_weights_q_noalloc, nat.lib().aih_qgemm):
+            yb.write(np.full(m * n + 8, -7.0, np.float32))
+            nat.check(fn(device.handle, int(qtype), wb.get_pointer(), n, k, xb.get_pointer(), m,
+                         yb.get_pointer() + offset), "GEMM")
+            all_ = yb.read_range(0, m * n + 8, np.float32)
+            at = offset // 4
+            assert np.all(all_[:at] == -7.0) and np.all(all_[at + m * n:] == -7.0)   # nothing outside Y
+            got.append(all_[at:at + m * n].reshape(m, n))
+    finally:
+        for b in (wb, xb, yb):
+            b.dispose()
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    assert_close(got[0], orc.matvec(qtype, w, n, k, x, nthreads=16), TOL, "type %d %dx%d M=%d" % (qtype, n, k, m))
+
+
 def test_subnormal_scales(device, orc):
     rng = np.random.default_rng(9)
     n, k, m = 70, 512, 33

@@ -156,6 +156,15 @@ def test_silu_pairs_operand_chain_equals_separate_operators(device, d, f, m, qt_
             b.dispose()
 
 
+# the same with K split over workgroups (at most 256 rows, few tiles): the
+# summing pass writes the operand image
+@pytest.mark.parametrize("m", [9, 64, 200])
+def test_silu_pairs_operand_chain_with_split_k(device, m):
+    if device.info().compute_units == 256:
+        assert nat.qgemm_plan(device.handle, 640, 4096, m)[1] > 1
+    test_silu_pairs_operand_chain_equals_separate_operators(device, 4096, 320, m, nat.Q8_0)
+
+
 def test_qgemm_fused_argument_errors(device):
     L, h = nat.lib(), device.handle
     n, k, m = 64, 256, 16
@@ -240,6 +249,15 @@ def test_qkv_rope_gemm_equals_gemm_then_rope(device, nh, nkv, k, m, start, dpos,
     finally:
         for b_ in bufs + [tb, pb]:
             b_.dispose()
+
+
+# the same with K split over workgroups: the summing pass rotates and stores,
+# inside the table and the cache and past the end of either
+@pytest.mark.parametrize("m,start,dpos,trows,crows", [(9, 0, None, 64, 64), (100, 20, 5, 160, 110), (256, 0, 30, 200, 300)])
+def test_qkv_rope_gemm_with_split_k(device, m, start, dpos, trows, crows):
+    if device.info().compute_units == 256:
+        assert nat.qgemm_plan(device.handle, 1024, 4096, m)[1] > 1
+    test_qkv_rope_gemm_equals_gemm_then_rope(device, 4, 2, 4096, m, start, dpos, trows, crows, nat.PRE_RMSNORM, nat.Q4_K)
 
 
 def test_qkv_rope_gemm_argument_errors(device):
