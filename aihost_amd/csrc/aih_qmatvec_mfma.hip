@@ -33,6 +33,8 @@
 // sub-block t and zeros elsewhere (read from an all-zero LDS row).  So every
 // output element belongs to exactly one (column, sub-block), and lane l holds
 // rows 4(l/16)..+3 of weight row l%16: the very row whose header it decoded.
+// Q8_0 and Q4_0 order the rows and the elements so that a lane's rows are its
+// own blocks' (UQ80, below).
 //
 // Work split.  K is cut into 256-element units (one Q4_K/Q6_K super-block,
 // eight Q8_0/Q4_0 blocks).  A workgroup of four waves owns 64 weight rows (a
@@ -40,7 +42,8 @@
 // In each round of up to UPW units the workgroup stages its slice of X
 // (all columns) into LDS as hi/lo fp16 pieces, with the per-group scales and
 // the per-sub-block sums of x, and each lane loads, for its weight row, the
-// 8 codes of every 32-element window that its k-block covers.  Each workgroup
+// 8 codes of every 32-element window that its k-block covers (Q4_K, Q6_K) or
+// two whole blocks of the unit (Q8_0, Q4_0).  Each workgroup
 // writes its 64 x batch partial sums to the context workspace (or to the
 // staging memory the allocation-free entry point supplies); a second
 // kernel adds the splits in a fixed order (the result does not depend on
@@ -76,18 +79,20 @@ __device__ __forceinline__ uint64_t bld8(Rsrc r, uint32_t vo, uint32_t so)
     const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, vo, so, 0);
     return (uint64_t)v[0] | ((uint64_t)v[1] << 32);
 }
-// The 8 bytes at vo + 2 for a 4-byte-aligned vo (Q8_0/Q4_0 code pieces that
-// start at 2 mod 4): one aligned 12-byte load and two funnel shifts; an
-// 8-byte load at 2 mod 4 takes the slow unaligned path.
-__device__ __forceinline__ uint64_t bld8_at2(Rsrc r, uint32_t vo, uint32_t so)
+__device__ __forceinline__ uint32_t bld4(Rsrc r, uint32_t vo, uint32_t so)
 {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b96(r, vo, so, 0);
-    const uint32_t lo = __builtin_amdgcn_alignbit(v[1], v[0], 16), hi = __builtin_amdgcn_alignbit(v[2], v[1], 16);
-    return (uint64_t)lo | ((uint64_t)hi << 32);
+    return __builtin_amdgcn_raw_buffer_load_b32(r, vo, so, 0);
 }
 __device__ __forceinline__ uint32_t bld2(Rsrc r, uint32_t vo, uint32_t so)
 {
     return __builtin_amdgcn_raw_buffer_load_b16(r, vo, so, 0);
+}
+__device__ __forceinline__ void put4(uint32_t *to, u4 v)
+{
+    to[0] = v.x;
+    to[1] = v.y;
+    to[2] = v.z;
+    to[3] = v.w;
 }
 __device__ __forceinline__ float f16_bits(uint32_t v)
 {
@@ -136,10 +141,11 @@ __device__ constexpr int kPerm[8] = {0, 2, 1, 3, 4, 6, 5, 7};
 // so window w = sub-block w, and lane q reads qs[32g + 8q .. +7] for g < 4.
 struct UQ4K {
     static constexpr int kBytes = 144, kBlocks = 1, kBlockElems = 256, SB = 32;
+    static constexpr bool kOwner = false;
     static constexpr bool kOwnMin = true;       // o independent of k
     static constexpr float kSumScale = 1.f;
     struct Raw { u4 hdr; uint64_t qs[4]; };
-    __device__ static void load(Rsrc r, uint32_t rowoff, int q, uint32_t so, int, Raw &w)
+    __device__ static void load(Rsrc r, uint32_t rowoff, int q, uint32_t so, Raw &w)
     {
         w.hdr = bld16(r, rowoff, so);
 #pragma unroll
@@ -160,7 +166,7 @@ struct UQ4K {
             o[j] = dmin * (float)mn;
         }
     }
-    __device__ static h8 code(const Raw &r, int w, int)
+    __device__ static h8 code(const Raw &r, int w)
     {
         // the low (even w) or high nibble of each byte, as 64c
         const uint64_t v = r.qs[w >> 1];
@@ -177,10 +183,11 @@ struct UQ4K {
 // scales and d.
 struct UQ6K {
     static constexpr int kBytes = 210, kBlocks = 1, kBlockElems = 256, SB = 16;
+    static constexpr bool kOwner = false;
     static constexpr bool kOwnMin = false;      // o = 32 d sc = 512 k
     static constexpr float kSumScale = -512.f;
     struct Raw { uint64_t ql[4], qh[2]; u4 sc; uint32_t d; };
-    __device__ static void load(Rsrc r, uint32_t rowoff, int q, uint32_t so, int, Raw &w)
+    __device__ static void load(Rsrc r, uint32_t rowoff, int q, uint32_t so, Raw &w)
     {
         // Units are 210 bytes: an odd unit starts at 2 mod 4 (rows at
         // multiples of 4).  Its pieces come from aligned loads 2 bytes lower,
@@ -208,7 +215,7 @@ struct UQ6K {
 #pragma unroll
         for (int j = 0; j < 16; ++j) k[j] = d16 * (float)(int)__builtin_amdgcn_sbfe((int)s[j >> 2], 8 * (j & 3), 8);
     }
-    __device__ static h8 code(const Raw &r, int w, int)
+    __device__ static h8 code(const Raw &r, int w)
     {
         const int h = w >> 2, Q = w & 3;
         const uint64_t l = r.ql[2 * h + (Q & 1)], hb = r.qh[h];
@@ -223,71 +230,91 @@ struct UQ6K {
     }
 };
 
-// Q8_0 unit = 8 blocks (d, qs[32] int8): window w = block w; lane q reads
-// qs[8q .. +7] of every block and the 8 scales.  Codes biased by 128 (xor
-// 0x80) are unsigned.
+// Q8_0 and Q4_0: the unit is 8 blocks of 34 or 18 bytes, each a sub-block with
+// its own scale.  Reading every block in 8-byte pieces took 16 loads of a
+// lane per unit, half of them off their natural alignment, and the vector
+// memory path, not HBM, bounded the kernel.  Here lane q owns blocks 2q and
+// 2q + 1 of its row's unit and reads their 68 or 36 bytes in 16-byte loads
+// and one dword, at multiples of 4 bytes (rows and units start there: K is a
+// multiple of 64).  Group g (of 2) contracts block 2t + g of every t < 4, in
+// four windows: in window j lane q holds elements 8j .. 8j + 7 of block
+// 2q + g, so its activations all belong to sub-block t = q.  5..8 columns take
+// two tiles of four columns that share the codes.
+// On MI355X per call (pieces of 8 bytes -> owned pairs of blocks): Q4_0 14336 x
+// 4096 4 columns 32.9 -> 13.5 us, 8 columns 32.1 -> 18.2, 32000 x 14336 x 8
+// 262 -> 129; Q8_0 14336 x 4096 x 4 30.8 -> 16.5, 4096 x 14336 x 8 35.7 ->
+// 25.9.  Runs of four blocks shared by two lanes in one 8-column tile (half
+// the MFMAs, every byte loaded twice) measured 18.8, 161 and 29.6 us at the
+// 8-column sizes.
+// In a last, partial unit (nb blocks inside the row) single dwords are read,
+// so that a read past the tile's rows returns zeros on its own, and blocks
+// past the row get scale 0 (their activations are staged as zeros).
+template <int NW>
+struct PairRaw { uint32_t w[NW]; uint32_t nb; };
+
+template <int NW, bool WHOLE>
+__device__ __forceinline__ void load_pair(Rsrc r, uint32_t rowoff, int q, uint32_t so, int nb, PairRaw<NW> &w)
+{
+    const uint32_t at = rowoff + 4 * NW * q;
+    w.nb = WHOLE ? 8u : (uint32_t)nb;
+    if constexpr (WHOLE) {
+#pragma unroll
+        for (int i = 0; i < NW / 4; ++i) put4(w.w + 4 * i, bld16(r, at + 16 * i, so));
+        w.w[NW - 1] = bld4(r, at + 4 * (NW - 1), so);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NW; ++i) w.w[i] = bld4(r, at + 4 * i, so);
+    }
+}
+// Dwords i and i + 1 of the codes of block g (at byte 2 of the pair, or at the
+// dword after its middle), and its scale times f.
+template <int NW>
+__device__ __forceinline__ void pair_codes(const PairRaw<NW> &r, int g, int i, uint32_t &a, uint32_t &b)
+{
+    if (g) {
+        a = r.w[NW / 2 + 1 + i];
+        b = r.w[NW / 2 + 2 + i];
+    } else {
+        a = __builtin_amdgcn_alignbit(r.w[i + 1], r.w[i], 16);
+        b = __builtin_amdgcn_alignbit(r.w[i + 2], r.w[i + 1], 16);
+    }
+}
+template <int NW>
+__device__ __forceinline__ float pair_scale(const PairRaw<NW> &r, int q, int g, float f)
+{
+    return (uint32_t)(2 * q + g) < r.nb ? f * f16_bits(g ? r.w[NW / 2] >> 16 : r.w[0]) : 0.f;
+}
+
+// Q8_0 block: d, qs[32] int8.  Codes biased by 128 (xor 0x80) are unsigned.
 struct UQ80 {
     static constexpr int kBytes = 272, kBlocks = 8, kBlockElems = 32, SB = 32;
+    static constexpr bool kOwner = true;
     static constexpr bool kOwnMin = false;      // o = 128 d = 512 k
-    static constexpr float kSumScale = -512.f;
-    struct Raw { uint64_t qs[8]; uint32_t d[8]; };
-    __device__ static void load(Rsrc r, uint32_t rowoff, int q, uint32_t so, int nb, Raw &w)
+    static constexpr float kSumScale = -512.f, kScale = 0.25f;   // codes enter as 4(c + 128)
+    static constexpr int kDwords = 17;
+    typedef PairRaw<kDwords> Raw;
+    __device__ static h8 code(const Raw &r, int g, int j)
     {
-        // a block past the row's end (only in a last, partial unit) re-reads
-        // the start of the unit, so no read leaves the row, and gets scale 0.
-        // Rows and units start at multiples of 4 bytes (K is a multiple of
-        // 64): the pieces of even blocks lie at 2 mod 4, those of odd ones
-        // are aligned.
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const uint32_t o = b < nb ? rowoff + 34 * b : rowoff;
-            if (b % 2 == 0) w.qs[b] = bld8_at2(r, o + 8 * q, so);
-            else w.qs[b] = bld8(r, b < nb ? o + 2 + 8 * q : o + 8 * q, so);
-            w.d[b] = b < nb ? bld2(r, o, so) : 0u;
-        }
-    }
-    __device__ static void coef(const Raw &r, float *k, float *)
-    {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) k[j] = 0.25f * f16_bits(r.d[j]);   // codes enter as 4(c + 128)
-    }
-    __device__ static h8 code(const Raw &r, int w, int)
-    {
-        const uint64_t v = r.qs[w] ^ 0x8080808080808080ull;
-        return frag((uint32_t)v, (uint32_t)(v >> 32), 2, 6, 0x03FC03FCu);
+        uint32_t a, b;
+        pair_codes(r, g, 2 * j, a, b);
+        return frag(a ^ 0x80808080u, b ^ 0x80808080u, 2, 6, 0x03FC03FCu);
     }
 };
 
-// Q4_0 unit = 8 blocks (d, qs[16]): in block w, elements j < 16 are the low
-// nibbles of qs[j], elements 16 + j the high nibbles; lane q reads
-// qs[8(q%2) .. +7] and takes the low (q < 2) or high (q >= 2) nibbles.
+// Q4_0 block: d, qs[16]; elements j < 16 are the low nibbles of qs[j], elements
+// 16 + j the high nibbles.
 struct UQ40 {
     static constexpr int kBytes = 144, kBlocks = 8, kBlockElems = 32, SB = 32;
+    static constexpr bool kOwner = true;
     static constexpr bool kOwnMin = false;      // o = 8 d = 512 k
-    static constexpr float kSumScale = -512.f;
-    struct Raw { uint64_t qs[8]; uint32_t d[8]; };
-    __device__ static void load(Rsrc r, uint32_t rowoff, int q, uint32_t so, int nb, Raw &w)
+    static constexpr float kSumScale = -512.f, kScale = 0.015625f;   // codes enter as 64c
+    static constexpr int kDwords = 9;
+    typedef PairRaw<kDwords> Raw;
+    __device__ static h8 code(const Raw &r, int g, int j)
     {
-        // as Q8_0: even blocks' pieces at 2 mod 4, odd ones aligned
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const uint32_t o = b < nb ? rowoff + 18 * b : rowoff;
-            if (b % 2 == 0) w.qs[b] = bld8_at2(r, o + 8 * (q & 1), so);
-            else w.qs[b] = bld8(r, b < nb ? o + 2 + 8 * (q & 1) : o + 8 * (q & 1), so);
-            w.d[b] = b < nb ? bld2(r, o, so) : 0u;
-        }
-    }
-    __device__ static void coef(const Raw &r, float *k, float *)
-    {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) k[j] = 0.015625f * f16_bits(r.d[j]);   // codes enter as 64c
-    }
-    __device__ static h8 code(const Raw &r, int w, int q)
-    {
-        // low nibbles for lanes q < 2, high nibbles for q >= 2, both as 64c
-        const uint64_t v = r.qs[w];
-        return q >= 2 ? frag((uint32_t)v, (uint32_t)(v >> 32), 2, 6, 0x03C003C0u)
-                      : frag((uint32_t)v, (uint32_t)(v >> 32), 6, 2, 0x03C003C0u);
+        uint32_t a, b;
+        pair_codes(r, g, 2 * (j & 1), a, b);
+        return j >= 2 ? frag(a, b, 2, 6, 0x03C003C0u) : frag(a, b, 6, 2, 0x03C003C0u);
     }
 };
 
@@ -346,7 +373,7 @@ struct Img {
 // tid + 256 j of the round is column c / (32 R), elements 8 (c % (32 R)) ..
 // +7, at byte offset xo[j] + 1024 ub in xr.  lead: a previous round of this
 // workgroup may still be reading the image.
-template <class U, int T, int R, bool WHOLE>
+template <class U, int T, int CB, int R, bool WHOLE>
 __device__ __forceinline__ void round_of(Rsrc wr, uint32_t rowoff, Rsrc xr, const uint32_t *xo, int ub, int nb,
                                          int64_t K, int batch, Img<R, T * U::SB, U::SB> &im, bool lead, int tid,
                                          int q, const int *xrow, float *out)
@@ -366,7 +393,11 @@ __device__ __forceinline__ void round_of(Rsrc wr, uint32_t rowoff, Rsrc xr, cons
     __builtin_amdgcn_sched_barrier(0);
     typename U::Raw rw[R];
 #pragma unroll
-    for (int u = 0; u < R; ++u) U::load(wr, rowoff, q, (uint32_t)(ub + u) * U::kBytes, WHOLE ? U::kBlocks : nb, rw[u]);
+    for (int u = 0; u < R; ++u) {
+        const uint32_t so = (uint32_t)(ub + u) * U::kBytes;
+        if constexpr (U::kOwner) load_pair<U::kDwords, WHOLE>(wr, rowoff, q, so, nb, rw[u]);
+        else U::load(wr, rowoff, q, so, rw[u]);
+    }
     __builtin_amdgcn_sched_barrier(0);
     if (lead) lds_barrier();
     if constexpr (!WHOLE) {
@@ -418,6 +449,41 @@ __device__ __forceinline__ void round_of(Rsrc wr, uint32_t rowoff, Rsrc xr, cons
     }
     lds_barrier();
     __builtin_amdgcn_sched_barrier(0);   // keep the codes and MFMAs after the barrier
+    if constexpr (U::kOwner) {
+        // lane (n, q): MFMA rows i = 4q + r = sub-block q of column 4h + r in
+        // the tile of column half h
+        constexpr int CH = CB / 4;
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            float k[2], fv[CB], sv[CB][2];
+#pragma unroll
+            for (int g = 0; g < 2; ++g) k[g] = pair_scale(rw[u], q, g, U::kScale);
+#pragma unroll
+            for (int b = 0; b < CB; ++b) {
+                fv[b] = im.f[b][u * NGU + q / 2];   // both blocks of the lane in one staged group
+#pragma unroll
+                for (int g = 0; g < 2; ++g) sv[b][g] = im.sx[b][u * 8 + 2 * q + g];
+            }
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                f4 acc[CH] = {};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const h8 c = U::code(rw[u], g, j);
+                    const int piece = u * 32 + 8 * q + 4 * g + j;
+#pragma unroll
+                    for (int h = 0; h < CH; ++h) {
+                        acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(im.lo[xrow[h]][piece], c, acc[h], 0, 0, 0);
+                        acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(im.hi[xrow[h]][piece], c, acc[h], 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int b = 0; b < CB; ++b)   // o = -kSumScale * k: the staged sums carry the factor
+                    out[b] = __builtin_fmaf(k[g], __builtin_fmaf(acc[b / 4][b % 4], fv[b], sv[b][g]), out[b]);
+            }
+        }
+        return;
+    } else {
     // lane (n, q'): MFMA rows i = 4q' + r, i.e. column q' * NB + r / T and
     // sub-block r % T of each group
     constexpr int NB = 4 / T, NSB = UNIT / SB;
@@ -443,7 +509,7 @@ __device__ __forceinline__ void round_of(Rsrc wr, uint32_t rowoff, Rsrc xr, cons
 #pragma unroll
             for (int wg = 0; wg < WPG; ++wg) {
                 const int w = g * WPG + wg;
-                const h8 c = U::code(rw[u], w, q);
+                const h8 c = U::code(rw[u], w);
                 const int piece = u * 32 + w * 4 + q;
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(im.lo[xrow[wg]][piece], c, acc, 0, 0, 0);
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(im.hi[xrow[wg]][piece], c, acc, 0, 0, 0);
@@ -460,13 +526,14 @@ __device__ __forceinline__ void round_of(Rsrc wr, uint32_t rowoff, Rsrc xr, cons
             }
         }
     }
+    }
 }
 
 // Workgroup g: row tile g % ntiles, split g / ntiles, units [split * per,
 // min(nunits, (split + 1) * per)) in rounds of UPW units (then single units).
 // P != nullptr: partial sums of the split to P[(split * batch + b) * np + n];
 // else Y directly.
-template <class U, int T, int UPW>
+template <class U, int T, int CB, int UPW>
 __global__ void __launch_bounds__(TW * 64)
 qmv_split_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes, const float *__restrict__ X,
                  int64_t ldx, int batch, int ntiles, int per, float *__restrict__ P, int64_t np,
@@ -502,13 +569,17 @@ qmv_split_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes, cons
         const int col = tid / 32, kc = tid % 32;
         xo1[0] = (uint32_t)(((int64_t)min(col, batch - 1) * ldx + 8 * kc) * 4);
     }
-    // MFMA row i = n16 of this lane's A fragments: (column i / T, sub-block
-    // i % T); in window wg of a group it reads its column's activations when
-    // lane q's 8 elements lie in sub-block i % T, else the zero row
+    // MFMA row i = n16 of this lane's A fragments.  Owner formats: sub-block
+    // i / 4 of column i % 4 + 4h in the tile of column half h, read where the
+    // sub-block is the lane's own.  Else (column i / T, sub-block i % T), read
+    // in window wg of a group when lane q's 8 elements lie in sub-block i % T.
+    // Elsewhere the lane reads the zero row.
     int xrow[WPG];
+    static_assert(!U::kOwner || (T == 4 && WPG == 4 && CB <= 8), "owner formats: four sub-blocks per tile");
 #pragma unroll
     for (int wg = 0; wg < WPG; ++wg) {
-        const int b = n16 / T, t = n16 % T, s = (32 * wg + 8 * q) / SB;
+        const int b = U::kOwner ? n16 % 4 + 4 * wg : n16 / T, t = U::kOwner ? n16 / 4 : n16 % T;
+        const int s = U::kOwner ? q : (32 * wg + 8 * q) / SB;
         xrow[wg] = (s == t && b < batch) ? b : ZROW;
     }
     // the zero row of the image (never written by the staging)
@@ -517,19 +588,32 @@ qmv_split_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes, cons
         im.lo[ZROW][p] = h8{};
     }
 
-    float out[4] = {0.f, 0.f, 0.f, 0.f};
+    float out[U::kOwner ? CB : 4] = {};
     int ub = ua;
     for (; ub + UPW <= ue_whole; ub += UPW)
-        round_of<U, T, UPW, true>(wr, rowoff, xr, xo, ub, U::kBlocks, K, batch, im, ub != ua, tid, q, xrow, out);
+        round_of<U, T, CB, UPW, true>(wr, rowoff, xr, xo, ub, U::kBlocks, K, batch, im, ub != ua, tid, q, xrow, out);
     for (; ub < ue; ++ub) {
         const int nb = (int)min<int64_t>(U::kBlocks, nblk - (int64_t)ub * U::kBlocks);
-        round_of<U, T, 1, false>(wr, rowoff, xr, xo1, ub, nb, K, batch,
+        round_of<U, T, CB, 1, false>(wr, rowoff, xr, xo1, ub, nb, K, batch,
                                  *reinterpret_cast<Img<1, G, SB> *>(&im), ub != ua, tid, q, xrow, out);
     }
 
+    const int64_t n = row0 + 16 * wave + n16;
+    if constexpr (U::kOwner) {
+        // out[b]: column b over the lane's own blocks; add the four lanes of a row
+#pragma unroll
+        for (int b = 0; b < CB; ++b) {
+            out[b] += __shfl_xor(out[b], 16);
+            out[b] += __shfl_xor(out[b], 32);
+            if (n < N && q == b % 4 && b < batch) {
+                if (P) P[((int64_t)split * batch + b) * np + n] = out[b];
+                else Y[(int64_t)b * ldy + n] = out[b];
+            }
+        }
+        return;
+    }
     // out[r] = row 4q + r = (column (4q + r) / T, sub-block (4q + r) % T) of
     // weight row n16: add the sub-blocks of each column
-    const int64_t n = row0 + 16 * wave + n16;
     if (n < N) {
 #pragma unroll
         for (int r = 0; r < 4; r += T < 4 ? T : 4) {
@@ -569,7 +653,7 @@ split_sum_kernel(const float *__restrict__ P, int64_t np, int S, int batch, int6
     Y[(int64_t)col * ldy + n] = s;
 }
 
-template <class U, int T>
+template <class U, int T, int CB>
 int launch_t(aih_ctx *ctx, const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
              const float *X, int64_t ldx, float *Y, int64_t ldy, int batch, const aih_scratch *ext)
 {
@@ -612,13 +696,13 @@ int launch_t(aih_ctx *ctx, const uint8_t *W, int64_t N, int64_t K, int64_t row_b
     const dim3 grid((unsigned)(ntiles * S)), block(TW * 64);
     const int nt = (int)ntiles, pr = (int)per;
     if (per >= 4)
-        hipLaunchKernelGGL((qmv_split_kernel<U, T, 4>), grid, block, 0, ctx->stream,
+        hipLaunchKernelGGL((qmv_split_kernel<U, T, CB, 4>), grid, block, 0, ctx->stream,
                            W, N, K, row_bytes, X, ldx, batch, nt, pr, P, np, Y, ldy);
     else if (per >= 2)
-        hipLaunchKernelGGL((qmv_split_kernel<U, T, 2>), grid, block, 0, ctx->stream,
+        hipLaunchKernelGGL((qmv_split_kernel<U, T, CB, 2>), grid, block, 0, ctx->stream,
                            W, N, K, row_bytes, X, ldx, batch, nt, pr, P, np, Y, ldy);
     else
-        hipLaunchKernelGGL((qmv_split_kernel<U, T, 1>), grid, block, 0, ctx->stream,
+        hipLaunchKernelGGL((qmv_split_kernel<U, T, CB, 1>), grid, block, 0, ctx->stream,
                            W, N, K, row_bytes, X, ldx, batch, nt, pr, P, np, Y, ldy);
     int st = aih_launch_status();
     if (st != AIH_OK || !P) return st;
@@ -628,13 +712,14 @@ int launch_t(aih_ctx *ctx, const uint8_t *W, int64_t N, int64_t K, int64_t row_b
     return aih_launch_status();
 }
 
-// 3..4 columns: four sub-blocks per column in the 16 MFMA rows; 5..8: two
+// 3..4 columns: four sub-blocks per column in the 16 MFMA rows; 5..8: two, or
+// for the owner formats four again and two tiles
 template <class U>
 int launch(aih_ctx *ctx, const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
            const float *X, int64_t ldx, float *Y, int64_t ldy, int batch, const aih_scratch *ext)
 {
-    return batch <= 4 ? launch_t<U, 4>(ctx, W, N, K, row_bytes, X, ldx, Y, ldy, batch, ext)
-                      : launch_t<U, 2>(ctx, W, N, K, row_bytes, X, ldx, Y, ldy, batch, ext);
+    return batch <= 4 ? launch_t<U, 4, 4>(ctx, W, N, K, row_bytes, X, ldx, Y, ldy, batch, ext)
+                      : launch_t<U, U::kOwner ? 4 : 2, 8>(ctx, W, N, K, row_bytes, X, ldx, Y, ldy, batch, ext);
 }
 
 }  // namespace

@@ -89,6 +89,20 @@ def test_edge_shapes(device, orc, qtype, n, k, batch):
     assert_close(y, ref, TOL, "type %d %dx%d b%d" % (qtype, n, k, batch))
 
 
+# 3..8 columns of the 32-element formats (one tile of four columns or two): a
+# lane owns two of the 8 blocks of a 256-element unit; K ending after 2, 4 or 6
+# blocks of a unit, one unit, rounds of several units and a rest; rows not
+# filling a tile.
+@pytest.mark.parametrize("batch", [3, 4, 5, 8])
+@pytest.mark.parametrize("n,k", [(1, 64), (17, 128), (64, 192), (65, 256), (130, 1344), (16, 4160), (96, 8192)])
+@pytest.mark.parametrize("qtype", [nat.Q8_0, nat.Q4_0])
+def test_block_pairs_of_the_small_batch_kernel(device, orc, qtype, n, k, batch):
+    w = synth_weight(qtype, n, k, seed=n + k)
+    x = x_of(k, batch, seed=batch + n)
+    assert_close(qmatvec(device, qtype, w, n, k, x), orc.matvec(qtype, w, n, k, x), TOL,
+                 "type %d %dx%d b%d" % (qtype, n, k, batch))
+
+
 @pytest.mark.parametrize("qtype,n,k,batch", [
     (nat.Q8_0, 140001, 64, 2),     # more rows than one launch holds (64 row groups per workgroup)
     (nat.Q4_K, 140001, 256, 1),
