@@ -486,64 +486,80 @@ qgemm_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
 }
 
 // Wide tiles for large products: a workgroup of eight waves owns a 256 MB (M)
-// x 64 (N) tile (MB = 1 or 2), so each dequantized weight feeds 2 MB times as
-// many outputs as in qgemm_kernel.  Every wave takes both roles in each
+// x 64 NB (N) tile (MB, NB = 1 or 2), so each dequantized weight feeds 2 MB
+// times as many outputs as in qgemm_kernel.  Every wave takes both roles in each
 // super-step s:
-//   - it dequantizes its 8 of the 64 weight rows (row 8w + lane / 8) for
+//   - it dequantizes its 8 NB of the 64 NB weight rows (rows 64 i + 8w + lane / 8) for
 //     super-step s+1 into the other LDS buffer, 32 weights per lane
-//     (Piece32), from packed loads PR256 super-steps ahead;
+//     (Piece32), from packed loads PR256 (NB = 2: one) super-steps ahead;
 //   - it multiplies super-step s: wave w owns rows 32 MB w .. +32 MB - 1 of
-//     the M tile and all 64 columns (2 MB 32x32 accumulators: each A fragment
-//     feeds two, each B fragment MB), A fragments from the tiled X AD 64-k
+//     the M tile and all 64 NB columns (2 MB NB 32x32 accumulators: each A fragment
+//     feeds 2 NB, each B fragment MB), A fragments from the tiled X AD 64-k
 //     chunks ahead, B fragments from LDS.
 // The two waves of a SIMD (w and w + 4) run the two halves in opposite
 // orders, so that one dequantizes while the other multiplies.  On MI355X a
 // 256-row workgroup takes about 1.25 times as long as a 128-row one, for
 // twice the outputs.
+// With 64 columns every A fragment is loaded for two MFMAs, 64 bytes per clock
+// and CU through the vector L1 at the full MFMA rate, which is all it gives:
+// the 512 x 64 tile reaches half that rate.  The 512 x 128 tile (NB = 2) halves
+// those loads; its 128 accumulator registers leave room for A one 64-k chunk
+// and B one 16-k slice ahead.  Per call, Q4_K K = 4096: 14336 x 2048 291 -> 237
+// us, 28672 x 512 138 -> 121 us.  Left out one at a time (a copy, 237 us): the
+// A loads -26 us, the dequantization -36 us, both -55 us: what remains is the
+// MFMAs, and the last round of workgroups.
 constexpr int BM2 = 256;
 constexpr int PR256 = 2;
 
-template <class T, int MB, int AD>
+template <class T, int MB, int NB, int AD>
 __global__ void __launch_bounds__(512)
 qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
                 const _Float16 *__restrict__ Xt, int64_t M, float *__restrict__ Y, int epi,
                 float *__restrict__ P, int64_t zs, int ssper, aih_rope_qkv_args ra)
 {
     static_assert(SC % AD == 0, "A ring depth divides a super-step");
-    constexpr int PR = PR256;
+    constexpr int PR = NB == 1 ? PR256 : 1;
     typedef typename Piece32<T>::type Pc;
     typedef typename Pc::Raw Raw;
-    __shared__ __align__(16) _Float16 wsh[2][BN][LD2];
+    __shared__ __align__(16) _Float16 wsh[2][BN * NB][LD2];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t m0 = (int64_t)blockIdx.y * BM2 * MB, n0 = (int64_t)blockIdx.x * BN;
+    const int64_t m0 = (int64_t)blockIdx.y * BM2 * MB, n0 = (int64_t)blockIdx.x * (BN * NB);
     const int nch = (int)(K / 64);
     // split z of K (gridDim.z > 1: partial sums into P + z * zs): super-steps
     // ss0 .. ss0 + nss - 1; chunk indices below stay absolute
     const int ss0 = (int)blockIdx.z * ssper;
     const int nss = min(ssper, (nch + SC - 1) / SC - ss0);
 
-    // dequantization share: row 8 wave + rl, 32 weights per lane (chunk pc, half ph)
+    // dequantization share: rows 64 i + 8 wave + rl, 32 weights per lane (chunk pc, half ph)
     const int rl = lane >> 3, p = lane & 7, pc = p >> 1, ph = p & 1;
-    const int64_t wn = n0 + 8 * wave + rl;
-    const uint8_t *wrow = W + (wn < N ? wn : N - 1) * row_bytes;
+    const uint8_t *wrow[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        const int64_t wn = n0 + 64 * i + 8 * wave + rl;
+        wrow[i] = W + (wn < N ? wn : N - 1) * row_bytes;
+    }
     auto gload = [&](int ss, Raw *r) {
         int c = (ss0 + ss) * SC + pc;
         c = c < nch ? c : nch - 1;
-        Pc::load(wrow, c, ph, r[0]);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) Pc::load(wrow[i], c, ph, r[i]);
     };
     // chunks past K exist only in a last, partial super-step, staged as zeros
     auto stage = [&](auto tail, int ss, int buf, const Raw *r) {
         const int c = (ss0 + ss) * SC + pc;
-        h8 o[4];
-        Pc::piece(r[0], c, ph, o);
-        _Float16 *d = &wsh[buf][8 * wave + rl][0];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            *reinterpret_cast<h8 *>(d + 8 * Pc::swz(8 * pc + Pc::col(ph, q) / 8)) =
-                decltype(tail)::value && c >= nch ? h8{} : o[q];
+        for (int i = 0; i < NB; ++i) {
+            h8 o[4];
+            Pc::piece(r[i], c, ph, o);
+            _Float16 *d = &wsh[buf][64 * i + 8 * wave + rl][0];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<h8 *>(d + 8 * Pc::swz(8 * pc + Pc::col(ph, q) / 8)) =
+                    decltype(tail)::value && c >= nch ? h8{} : o[q];
+        }
     };
 
-    // multiplication share: rows 32 MB wave .. +32 MB - 1 of the M tile
+    // multiplication share: rows 32 MB wave .. +32 MB - 1 of the M tile, all columns
     const int fr = lane & 31, fk = 8 * (lane >> 5);
     const int64_t kc = K / 16, mblocks = (M + 31) / 32;
     const _Float16 *xa[MB];
@@ -565,7 +581,7 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
 #pragma unroll
             for (int kk = 0; kk < 4; ++kk) f.a[j][kk] = ldg<h8>(xa[j] + ((int64_t)kb * 4 + kk) * 512);
     };
-    f16v acc[MB][2] = {};
+    f16v acc[MB][2 * NB] = {};
     struct BF { h8 b0[4], b1[4]; };
     auto bload = [&](int buf, int t, BF &b) {
 #pragma unroll
@@ -584,14 +600,24 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
             }
     };
 
+    // NB = 2: the B fragments of one k16 slice u of a super-step (all 128
+    // columns), one slice ahead of their MFMAs
+    struct BS { h8 b[2 * NB]; };
+    auto bslice = [&](int buf, int u, BS &b) {
+#pragma unroll
+        for (int i = 0; i < 2 * NB; ++i)
+            b.b[i] = *reinterpret_cast<const h8 *>(&wsh[buf][32 * i + fr][8 * Pc::swz(2 * u + fk / 8)]);
+    };
+
     // Iteration it: products of super-step it from buffer it & 1, and, if
     // `more`, the dequantization of super-step it + 1 into the other buffer
     // from ring slot r, whose loads are then reissued for super-step
     // it + 1 + PR when `reload`.
-    Raw ring[PR][1];
+    Raw ring[PR][NB];
     AF f[AD];   // chunk g of the A operand in f[g % AD]
     constexpr int BD = MB == 1 ? 2 : 1;   // B chunks in registers (the next one loaded early when 2)
     BF bb[BD];
+    BS bs[2];
     // The two waves of a SIMD (w and w + 4) take the two halves in opposite
     // orders, so that one dequantizes while the other multiplies.
     const bool valu_first = wave < 4;
@@ -604,12 +630,32 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
             }
             __builtin_amdgcn_sched_barrier(0);
         };
-        if (BD == 2) bload(buf, 0, bb[0]);
+        if (NB == 1 && BD == 2) bload(buf, 0, bb[0]);
         if (valu_first) deq();
         // the multiplying half at raised wave priority, so that the SIMD
         // issues its MFMAs ahead of the other wave's dequantization when both
         // are ready (6144 x 4096 and 28672 x 4096 at M = 512: 2% faster)
         __builtin_amdgcn_s_setprio(1);
+        if constexpr (NB > 1) {
+            bslice(buf, 0, bs[0]);
+#pragma unroll
+            for (int u = 0; u < 4 * SC; ++u) {
+                if (u + 1 < 4 * SC) bslice(buf, u + 1, bs[(u + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                AF &a = f[(u >> 2) % AD];
+#pragma unroll
+                for (int i = 0; i < 2 * NB; ++i)
+#pragma unroll
+                    for (int j = 0; j < MB; ++j)
+                        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.a[j][u & 3], bs[u & 1].b[i], acc[j][i], 0, 0, 0);
+                // this slice's A fragments, AD chunks ahead
+                int kb = SC * (ss0 + it) + (u >> 2) + AD;
+                kb = kb < nch ? kb : nch - 1;
+#pragma unroll
+                for (int j = 0; j < MB; ++j) a.a[j][u & 3] = ldg<h8>(xa[j] + ((int64_t)kb * 4 + (u & 3)) * 512);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else
 #pragma unroll
         for (int t = 0; t < SC; ++t) {
             if (BD == 1)
@@ -652,32 +698,48 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
     for (int j = 0; j < MB; ++j) {
         int64_t mb = (m0 + 32 * (MB * wave + j)) / 32;
         mb = mb < mblocks ? mb : mblocks - 1;
-        undo_row_exp(acc[j][0], acc[j][1], ev[j], E, mb * 32, lane);
-    }
-    if (epi == kEpiSiluOperand) {
-        // after the last barrier the tile buffers are free
 #pragma unroll
-        for (int j = 0; j < MB; ++j) {
-            silu_pairs_operand(acc[j][0], acc[j][1], lane, m0 + 32 * (MB * wave + j), n0, M, N,
-                               reinterpret_cast<float *>(&wsh[0][0][0]) + wave * 32 * 36,
-                               reinterpret_cast<_Float16 *>(Y));
+        for (int i = 0; i < NB; ++i) undo_row_exp(acc[j][2 * i], acc[j][2 * i + 1], ev[j], E, mb * 32, lane);
+    }
+    // every 32 x 64 block b = j NB + i (row fragment j, column pair i) of the
+    // wave, unrolled by hand: the epilogues are too large for the pragma
+    auto each = [&](auto f) {
+        f(std::integral_constant<int, 0>{});
+        if constexpr (MB * NB > 1) f(std::integral_constant<int, 1>{});
+        if constexpr (MB * NB > 2) {
+            f(std::integral_constant<int, 2>{});
+            f(std::integral_constant<int, 3>{});
+        }
+    };
+    if (epi == kEpiSiluOperand) {
+        // after the last barrier the tile buffers are free (N is a multiple of 64)
+        each([&](auto bc) {
+            constexpr int b = decltype(bc)::value;
+            if (NB == 1 || n0 + 64 * (b % NB) < N)
+                silu_pairs_operand(acc[b / NB][2 * (b % NB)], acc[b / NB][2 * (b % NB) + 1], lane,
+                                   m0 + 32 * (MB * wave + b / NB), n0 + 64 * (b % NB), M, N,
+                                   reinterpret_cast<float *>(&wsh[0][0][0]) + wave * 32 * 36,
+                                   reinterpret_cast<_Float16 *>(Y));
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the block is read before it is rewritten
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
+        });
         return;
     }
     if (epi == kEpiRopeQKV) {   // never split here (the plan splits this epilogue over 128-row tiles only)
-#pragma unroll
-        for (int j = 0; j < MB; ++j) rope_qkv_tile(acc[j][0], acc[j][1], lane, m0 + 32 * (MB * wave + j), n0, M, N, Y, ra);
+        each([&](auto bc) {
+            constexpr int j = decltype(bc)::value / NB, i = decltype(bc)::value % NB;
+            rope_qkv_tile(acc[j][2 * i], acc[j][2 * i + 1], lane, m0 + 32 * (MB * wave + j), n0 + 64 * i, M, N, Y, ra);
+        });
         return;
     }
     // a split's partial sums are stored (the summing pass adds them into Y)
     float *const Pz = P ? P + (int64_t)blockIdx.z * zs : nullptr;
-#pragma unroll
-    for (int j = 0; j < MB; ++j)
-        store_tile(acc[j][0], acc[j][1], lane, m0 + 32 * (MB * wave + j), n0, M, N, Pz ? Pz : Y,
+    each([&](auto bc) {
+        constexpr int j = decltype(bc)::value / NB, i = decltype(bc)::value % NB;
+        store_tile(acc[j][2 * i], acc[j][2 * i + 1], lane, m0 + 32 * (MB * wave + j), n0 + 64 * i, M, N, Pz ? Pz : Y,
                    !Pz && epi == kEpiAccumulate);
+    });
 }
 
 // The sum of the splits' partial sums p[0], p[zs], ... (in that order).
@@ -836,18 +898,22 @@ operand_fixup_kernel(_Float16 *__restrict__ Xt, int64_t mpad, int64_t K)
     if (lane == 0) reinterpret_cast<int32_t *>(img + aih_operand::row_exp_offset(mpad, K))[m] += mn;
 }
 
-// The tiling of a GEMM: rows per workgroup tile (128, 256 or 512) and, for
+// The tiling of a GEMM: rows (128, 256 or 512) and columns (64; 128 for the
+// widest, never split) per workgroup tile and, for
 // 128- and 512-row tiles, the number of K splits (splits > 1: partial sums in
 // the second workspace, then a summing pass) of ssper super-steps each.
 struct GemmPlan {
     int tile = 128;
+    int cols = BN;
     int splits = 1;
     int ssper = 0;
 };
 
 // 256-row tiles halve the dequantization per output and 512-row tiles halve
 // it again; a workgroup of them takes about 1.25 and 2.35 times as long as
-// one of 128 rows (measured on MI355X).  The shape with the fewest such
+// one of 128 rows, one of 512 x 128 about 3.6 times (measured on MI355X;
+// chip full, all four formats: 112-127 us a round of 4096 of K, against 68-76
+// of 512 x 64; nearly empty 82 against 62).  The shape with the fewest such
 // rounds of workgroups over the device's CUs wins (ties to the smaller tile).
 // Costs in units of 1/20 of a 128-row workgroup.  Products of more than 256
 // rows whose 512-row tiles leave CUs idle split K over workgroups: S splits
@@ -916,6 +982,11 @@ GemmPlan plan_gemm(int64_t cu_count, int64_t N, int64_t K, int64_t M, int epi, b
         }
     }
     p.tile = c4 < c2 && c4 < c1 ? 512 : c2 < c1 ? 256 : 128;
+    const double c8 = 72 * rounds((N + 2 * BN - 1) / (2 * BN) * gy4);
+    if (c8 < std::min(c1, std::min(c2, c4))) {
+        p.tile = 512;
+        p.cols = 2 * BN;
+    }
     return p;
 }
 
@@ -976,11 +1047,14 @@ int launch(aih_ctx *ctx, const uint8_t *W, int64_t N, int64_t K, int64_t row_byt
     }
     float *const P = static_cast<float *>(ws);
     const unsigned gz = (unsigned)p.splits;
-    if (p.tile == 512)
-        hipLaunchKernelGGL((qgemm256_kernel<T, 2, 2>), dim3((unsigned)gx, (unsigned)gy4, gz), dim3(512), 0, ctx->stream,
+    if (p.tile == 512 && p.cols == 2 * BN)
+        hipLaunchKernelGGL((qgemm256_kernel<T, 2, 2, 1>), dim3((unsigned)((N + 2 * BN - 1) / (2 * BN)), (unsigned)gy4),
+                           dim3(512), 0, ctx->stream, W, N, K, row_bytes, Xh, M, Y, epi, P, zs, p.ssper, ra);
+    else if (p.tile == 512)
+        hipLaunchKernelGGL((qgemm256_kernel<T, 2, 1, 2>), dim3((unsigned)gx, (unsigned)gy4, gz), dim3(512), 0, ctx->stream,
                            W, N, K, row_bytes, Xh, M, Y, epi, P, zs, p.ssper, ra);
     else if (p.tile == 256)
-        hipLaunchKernelGGL((qgemm256_kernel<T, 1, SC>), dim3((unsigned)gx, (unsigned)gy2), dim3(512), 0, ctx->stream,
+        hipLaunchKernelGGL((qgemm256_kernel<T, 1, 1, SC>), dim3((unsigned)gx, (unsigned)gy2), dim3(512), 0, ctx->stream,
                            W, N, K, row_bytes, Xh, M, Y, epi, P, zs, p.ssper, ra);
     else
         hipLaunchKernelGGL((qgemm_kernel<T>), dim3((unsigned)gx, (unsigned)gy, gz), dim3(64 * (4 + GRing<T>::NP)), 0, ctx->stream,

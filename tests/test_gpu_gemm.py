@@ -132,6 +132,32 @@ def test_small_grid_split_k(device, orc, qtype, n, k, m, offset):
     assert_close(got[0], orc.matvec(qtype, w, n, k, x, nthreads=16), TOL, "type %d %dx%d M=%d" % (qtype, n, k, m))
 
 
+# The 512 x 128 tiles of large products: row and column remainders, a second
+# column half past N, 64-k remainders, one super-step.  A row's bits do not
+# depend on the tiling, so the product equals the one taken 300 rows at a time
+# (128-row tiles on a 256-CU device).
+@pytest.mark.parametrize("qtype,n,k,m", [(nat.Q4_K, 8150, 512, 1537), (nat.Q6_K, 14300, 768, 1000),
+                                         (nat.Q8_0, 28600, 192, 500), (nat.Q4_0, 8129, 1344, 2048)])
+def test_wide_tiles_equal_row_chunks(device, qtype, n, k, m):
+    if device.info().compute_units == 256:
+        assert nat.qgemm_plan(device.handle, n, k, m, may_split=False) == (512, 1)
+    wb, xb = upload(device, synth_weight(qtype, n, k, seed=n + k)), upload(device, x_of(m, k, seed=m))
+    yb, cb = device.create_buffer(m * n * 4 + 32), device.create_buffer(m * n * 4)
+    f = nat.lib().aih_matmul_weights_q
+    try:
+        yb.write(np.full(m * n + 8, -7.0, np.float32))
+        nat.check(f(device.handle, int(qtype), wb.get_pointer(), n, k, xb.get_pointer(), m, yb.get_pointer()), "wide")
+        for r in range(0, m, 300):
+            nat.check(f(device.handle, int(qtype), wb.get_pointer(), n, k, xb.get_pointer() + r * k * 4,
+                        min(300, m - r), cb.get_pointer() + r * n * 4), "rows")
+        y, c = yb.read_range(0, m * n + 8, np.float32), cb.read_range(0, m * n, np.float32)
+    finally:
+        for b in (wb, xb, yb, cb):
+            b.dispose()
+    assert np.all(y[m * n:] == -7.0) and np.isfinite(c).all()
+    assert np.array_equal(y[:m * n].view(np.uint32), c.view(np.uint32))
+
+
 def test_subnormal_scales(device, orc):
     rng = np.random.default_rng(9)
     n, k, m = 70, 512, 33

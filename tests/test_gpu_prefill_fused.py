@@ -260,6 +260,15 @@ def test_qkv_rope_gemm_with_split_k(device, m, start, dpos, trows, crows):
     test_qkv_rope_gemm_equals_gemm_then_rope(device, 4, 2, 4096, m, start, dpos, trows, crows, nat.PRE_RMSNORM, nat.Q4_K)
 
 
+# both fused epilogues over the 512 x 128 tiles (N = 6144 and 8064)
+def test_epilogues_of_the_wide_tiles(device):
+    if device.info().compute_units == 256:
+        assert nat.qgemm_plan(device.handle, 6144, 256, 2000) == (512, 1)
+        assert nat.qgemm_plan(device.handle, 8064, 256, 1537) == (512, 1)
+    test_qkv_rope_gemm_equals_gemm_then_rope(device, 32, 8, 256, 2000, 3, None, 2048, 2040, nat.PRE_RMSNORM, nat.Q4_K)
+    test_silu_pairs_operand_chain_equals_separate_operators(device, 256, 4032, 1537, nat.Q8_0)
+
+
 def test_qkv_rope_gemm_argument_errors(device):
     L, h = nat.lib(), device.handle
     wb = upload(device, synth_weight(nat.Q4_K, 1024, 256))
