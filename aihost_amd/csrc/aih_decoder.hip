@@ -29,6 +29,8 @@
 #include "aih_internal.h"
 #include "aih_operand.h"
 
+#include <cfloat>
+
 namespace {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
@@ -1209,6 +1211,11 @@ __device__ __forceinline__ f4 bld16(Rsrc r, uint32_t vo)
     return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(r, vo, 0, 0));
 }
 
+__device__ __forceinline__ fl2 bld8(Rsrc r, uint32_t vo)
+{
+    return __builtin_bit_cast(fl2, __builtin_amdgcn_raw_buffer_load_b64(r, vo, 0, 0));
+}
+
 __device__ __forceinline__ float xor_lanes_max(float v)   // over lanes l, l^16, l^32, l^48
 {
     v = fmaxf(v, __shfl_xor(v, 16));
@@ -1306,6 +1313,43 @@ __device__ __forceinline__ void store_operand4(_Float16 *Xt, int64_t K, int64_t 
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
     const int64_t slot = ((m >> 5) * (K / 16) + (k0 >> 4)) * 64 + (m & 31) + 32 * ((k0 >> 3) & 1);
     *reinterpret_cast<h4 *>(Xt + slot * 8 + (k0 & 7)) = h4{(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
+}
+
+// A row's output of one head (r: dims 16 db + 4 g) as the operand image: block
+// b of this head (columns 32 b .. +31 of the head, dims 16 db + 4 g with
+// db = 2b, 2b + 1) of row i is held by the four lanes g of the row; its
+// exponent comes from their maximum (aih_operand.h).  Rows past n_q, up to the
+// next multiple of 32, are zero.
+__device__ __forceinline__ void prefill_operand_rows(_Float16 *__restrict__ Xt, f4 (&r)[8], int64_t i, int64_t n_q,
+                                                     int64_t q_stride, int h, int g)
+{
+    if (i >= n_q)
+#pragma unroll
+        for (int db = 0; db < 8; ++db) r[db] = f4{0.f, 0.f, 0.f, 0.f};
+    int eb[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        float mx = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) mx = fmaxf(mx, fmaxf(fabsf(r[2 * b][q]), fabsf(r[2 * b + 1][q])));
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        eb[b] = aih_operand::block_exp(mx);
+    }
+    const int64_t mpad = aih_operand::mpad_of(n_q);
+    if (i < mpad) {
+#pragma unroll
+        for (int db = 0; db < 8; ++db) {
+            const int e = eb[db >> 1] == aih_operand::kZeroBlock ? 0 : eb[db >> 1];
+            store_operand4(Xt, q_stride, i, (int64_t)h * kHD + 16 * db + 4 * g,
+                           f4{ldexpf(r[db].x, e), ldexpf(r[db].y, e), ldexpf(r[db].z, e), ldexpf(r[db].w, e)});
+        }
+        char *const img = reinterpret_cast<char *>(Xt);
+        const int eg = g == 0 ? eb[0] : g == 1 ? eb[1] : g == 2 ? eb[2] : eb[3];
+        reinterpret_cast<int8_t *>(img + aih_operand::block_exp_offset(mpad, q_stride))[i * (q_stride / 32) + 4 * h + g] =
+            (int8_t)eg;
+        if (h == 0 && g == 0) reinterpret_cast<int32_t *>(img + aih_operand::row_exp_offset(mpad, q_stride))[i] = 0;
+    }
 }
 
 __global__ void __launch_bounds__(512, 1)
@@ -1493,36 +1537,319 @@ attn_prefill_kernel(const float *__restrict__ Q, int64_t ldq, const float *__res
                 *reinterpret_cast<f4 *>(O + i * q_stride + (int64_t)h * kHD + 16 * db + 4 * g) = r[db];
         return;
     }
-    // The operand image: block b of this head (columns 32 b .. +31 of the
-    // head, dims 16 db + 4 g with db = 2b, 2b + 1) of row i is held by the
-    // four lanes g of the row; its exponent comes from their maximum
-    // (aih_operand.h).  Rows past n_q, up to the next multiple of 32, are zero.
-    if (i >= n_q)
+    prefill_operand_rows(Xt, r, i, n_q, q_stride, h, g);
+}
+
+// One tile of one KV head in registers, as the 512 threads of a workgroup
+// load it: K thread (keys kt_key + 32i, dims 8 kt_ch .. +7), V thread (dims
+// 2 vt_dp, + 1 of the 8 keys of slots 32 vt_t + 8 vt_g .. +7); rows past
+// p_last are zeros.
+struct KVTile512 {
+    f4 kr[4];
+    fl2 vr[8];
+
+    __device__ __forceinline__ void load(const float *__restrict__ Kc, const float *__restrict__ Vc,
+                                         int64_t kv_stride, int kvh, int64_t j0, int64_t p_last, int tid)
+    {
+        // one buffer per tile over its rows up to p_last: the rows past it
+        // (all of them when p_last < j0, as for a position before the
+        // cache) load as zeros
+        const uint32_t row = (uint32_t)kv_stride * 4;
+        const int64_t valid = max<int64_t>(0, min<int64_t>(p_last + 1 - j0, kKT));
+        const uint32_t bytes = __builtin_amdgcn_readfirstlane((uint32_t)valid * row);
+        const int64_t base = j0 * kv_stride + kvh * kHD;
+        const Rsrc rk = make_rsrc(uniform_ptr(Kc + base), bytes), rv = make_rsrc(uniform_ptr(Vc + base), bytes);
+        const int kt_key = tid >> 4, kt_ch = tid & 15;
+        const int vt_t = tid >> 8, vt_g = (tid >> 6) & 3, vt_dp = tid & 63;
 #pragma unroll
-        for (int db = 0; db < 8; ++db) r[db] = f4{0.f, 0.f, 0.f, 0.f};
-    int eb[4];
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t at = (uint32_t)(kt_key + 32 * i) * row + 32 * kt_ch;
+            kr[2 * i] = bld16(rk, at);
+            kr[2 * i + 1] = bld16(rk, at + 16);
+        }
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
+        for (int e = 0; e < 8; ++e)
+            vr[e] = bld8(rv, (uint32_t)(32 * vt_t + 16 * (e / 4) + 4 * vt_g + e % 4) * row + 8 * vt_dp);
+    }
+
+    // this wave's max |K| and |V|, into tmax[0][w] and tmax[1][w]
+    __device__ __forceinline__ void wave_max(float (*tmax)[8], int lane, int w) const
+    {
+        float mk = 0.f, mv = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) mk = fmaxf(mk, fabsf(kr[i][u]));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) mv = fmaxf(mv, fmaxf(fabsf(vr[i].x), fabsf(vr[i].y)));
+        mk = xor_lanes_max(row16_max(mk));
+        mv = xor_lanes_max(row16_max(mv));
+        if (lane == 0) {
+            tmax[0][w] = mk;
+            tmax[1][w] = mv;
+        }
+    }
+
+    // this thread's split chunks into the padded LDS images (K hi, K lo,
+    // V^T hi, V^T lo from lds)
+    __device__ __forceinline__ void split_to_lds(int ek, int ev, int tid, _Float16 *lds) const
+    {
+        const int kt_key = tid >> 4, kt_ch = tid & 15;
+        const int vt_t = tid >> 8, vt_g = (tid >> 6) & 3, vt_dp = tid & 63;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            h8 hi, lo;
+            split8(kr[2 * i], kr[2 * i + 1], ek, hi, lo);
+            _Float16 *at = lds + (kt_key + 32 * i) * kRKH + 8 * kt_ch;
+            *reinterpret_cast<h8 *>(at) = hi;
+            *reinterpret_cast<h8 *>(at + kKT * kRKH) = lo;
+        }
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            h8 hi, lo;
+            split8(f4{vr[0][d], vr[1][d], vr[2][d], vr[3][d]}, f4{vr[4][d], vr[5][d], vr[6][d], vr[7][d]}, ev, hi,
+                   lo);
+            _Float16 *at = lds + 2 * kKT * kRKH + (2 * vt_dp + d) * kRVH + 32 * vt_t + 8 * vt_g;
+            *reinterpret_cast<h8 *>(at) = hi;
+            *reinterpret_cast<h8 *>(at + kHD * kRVH) = lo;
+        }
+    }
+};
+
+__device__ __forceinline__ int split_exp_of(const float (*tmax)[8], int which)
+{
+    float m = tmax[which][0];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) m = fmaxf(m, tmax[which][w]);
+    return split_exp(m);
+}
+
+// The same products for NB heads of one KV head at once, where that still
+// fills the CUs (prefill_pairs).  attn_prefill_kernel is bound by the splitting
+// of K and V into fp16 pairs (352 of 586 VALU instructions per wave and tile)
+// and by its LDS reads (64 KB per wave and tile for 96 MFMAs).  Here a
+// workgroup's eight waves share one image of a 64-key tile (each thread splits
+// half as much, and holds half as many rows in flight), and every K and V
+// fragment feeds the queries of NB heads.  Wave w of half h owns the queries
+// 16w .. 16w + 15 of each head and the keys 32h .. 32h + 31 of every tile (score
+// blocks 2h, 2h + 1, product step t = h); the halves merge at the end as above.
+// Two images in LDS, one barrier per tile.
+// On MI355X, NB = 2, 32 heads over 8: 2048 queries 188 -> 142 us, 1024 at
+// position 2000 215 -> 179, 2048 at 2000 492 -> 363; 3.45 us a tile and
+// workgroup against 2.45 for one head.  With NB = 1 it is 3-5% slower than
+// attn_prefill_kernel, which therefore stays for one head at a time.
+template <int NB>
+__global__ void __launch_bounds__(512, 1)
+attn_prefill_group_kernel(const float *__restrict__ Q, int64_t ldq, const float *__restrict__ Kc,
+                          const float *__restrict__ Vc, float *__restrict__ O, int64_t n_q, int32_t n_heads,
+                          int32_t n_kv_heads, int32_t start, const int32_t *pos, int32_t max_len, float scale,
+                          _Float16 *__restrict__ Xt)
+{
+    // two tile images of K hi, K lo, V^T hi, V^T lo
+    constexpr int kImage = 2 * kKT * kRKH + 2 * kHD * kRVH;
+    __shared__ __align__(16) _Float16 lds2[2][kImage];
+    __shared__ float tmax[2][2][8];   // [tile parity][K, V][wave]
+    const int tid = threadIdx.x, wave = tid >> 6, half = wave >> 2, lane = tid & 63, w = wave & 3;
+    const int h0 = NB * blockIdx.x;   // this workgroup's heads, of one KV head: h0 .. h0 + NB - 1
+    const int g = lane >> 4, c = lane & 15;
+    const int kvh = h0 / (n_heads / n_kv_heads);
+    const int64_t kv_stride = (int64_t)n_kv_heads * kHD, q_stride = (int64_t)n_heads * kHD;
+    const int32_t p0 = dev_pos(start, pos);
+    // query tiles longest first
+    const int64_t i0 = (int64_t)(gridDim.y - 1 - blockIdx.y) * kQTile;
+    // keys beyond the cache (a position past max_len) are never read
+    const int64_t p_last = min<int64_t>(p0 + min<int64_t>(i0 + kQTile, n_q) - 1, (int64_t)max_len - 1);
+    const int64_t n_kt = prefill_key_tiles(i0, n_q, p0, max_len);
+    // Q^T operand: query 16w + c, dims 32s + 8g .. +7, split with the row's
+    // power of two (rows past n_q read the last row, never stored)
+    h8 qh[NB][4], ql[NB][4];
+    int eq[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const float *qrow = Q + min<int64_t>(i0 + 16 * w + c, n_q - 1) * ldq + (int64_t)(h0 + b) * kHD + 8 * g;
+        f4 qv[8];
         float mx = 0.f;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) mx = fmaxf(mx, fmaxf(fabsf(r[2 * b][q]), fabsf(r[2 * b + 1][q])));
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        eb[b] = aih_operand::block_exp(mx);
+        for (int s = 0; s < 4; ++s) {
+            qv[2 * s] = *reinterpret_cast<const f4 *>(qrow + 32 * s);
+            qv[2 * s + 1] = *reinterpret_cast<const f4 *>(qrow + 32 * s + 4);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) mx = fmaxf(mx, fabsf(qv[i][u]));
+        eq[b] = split_exp(xor_lanes_max(mx));
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const hl2 v = split_f16(qv[2 * s + e / 4][e % 4], eq[b]);
+                qh[b][s][e] = v.x;
+                ql[b][s][e] = v.y;
+            }
     }
-    const int64_t mpad = aih_operand::mpad_of(n_q);
-    if (i < mpad) {
+    const int64_t qpos = p0 + min<int64_t>(i0 + 16 * w + c, n_q - 1);   // last key the query attends to
+    const float sl = scale * 1.44269504088896341f;                       // scale log2(e)
+    float m[NB], l[NB];
+    int A = 1 << 20;   // O accumulators hold 2^A O (lowered by the first tile)
+    f4 o[NB][8];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        m[b] = -FLT_MAX;   // finite: a half whose keys so far are all masked keeps weight 0
+        l[b] = 0.f;
+#pragma unroll
+        for (int db = 0; db < 8; ++db) o[b][db] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+
+    // tile t: its rows are loaded during tile t - 2, split into image t % 2
+    // with the exponents of its maxima at the start of tile t - 1 (one
+    // barrier per tile)
+    KVTile512 kv;
+    int ek = 0, ev = 0;
+    if (n_kt > 0) {
+        kv.load(Kc, Vc, kv_stride, kvh, 0, p_last, tid);
+        kv.wave_max(tmax[0], lane, wave);
+        __syncthreads();
+        ek = split_exp_of(tmax[0], 0);
+        ev = split_exp_of(tmax[0], 1);
+        kv.split_to_lds(ek, ev, tid, lds2[0]);
+        if (n_kt > 1) {
+            kv.load(Kc, Vc, kv_stride, kvh, kKT, p_last, tid);
+            kv.wave_max(tmax[1], lane, wave);
+        }
+        __syncthreads();
+    }
+    for (int64_t it = 0; it < n_kt; ++it) {
+        const int64_t j0 = kKT * it;
+        const _Float16 *const ksh = lds2[it & 1], *const vsh = ksh + 2 * kKT * kRKH;
+        int ek_next = 0, ev_next = 0;
+        if (it + 1 < n_kt) {
+            ek_next = split_exp_of(tmax[(it + 1) & 1], 0);
+            ev_next = split_exp_of(tmax[(it + 1) & 1], 1);
+            kv.split_to_lds(ek_next, ev_next, tid, lds2[(it + 1) & 1]);
+            if (it + 2 < n_kt) kv.load(Kc, Vc, kv_stride, kvh, j0 + 2 * kKT, p_last, tid);   // in flight
+        }
+
+        // S^T = K Q^T, this half's two blocks of 16 keys
+        f4 sc[NB][2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            f4 acc[NB] = {};
+            const int at = (32 * half + 16 * kb + c) * kRKH + 8 * g;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const h8 kh = *reinterpret_cast<const h8 *>(&ksh[at + 32 * s]);
+                const h8 kl = *reinterpret_cast<const h8 *>(&ksh[kKT * kRKH + at + 32 * s]);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[b][s], acc[b], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[b][s], acc[b], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[b][s], acc[b], 0, 0, 0);
+            }
+#pragma unroll
+            for (int b = 0; b < NB; ++b) sc[b][kb] = acc[b];
+        }
+        // t = score log2(e) (the powers of two undone exactly in the
+        // multiplier), causal mask, online softmax of query c in base 2
+        // (the half's keys past lim are masked)
+        const int lim = (int)max<int64_t>(min<int64_t>(qpos - j0, kKT), -1) - 32 * half;
+        const int An = min(A, ev + 15);
+        const float fa = ldexpf(1.f, max(An - A, -160));
+        A = An;
+        const int ep = An - ev;   // P'' = P 2^(A - ev) <= 2^15
+        h8 ph[NB], pl[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const float cs = ldexpf(sl, -(eq[b] + ek));
+            float mx = -INFINITY;
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float v = 16 * kb + 4 * g + r > lim ? -INFINITY : sc[b][kb][r] * cs;
+                    sc[b][kb][r] = v;
+                    mx = fmaxf(mx, v);
+                }
+            mx = xor_lanes_max(mx);
+            const float mn = fmaxf(m[b], mx), corr = __builtin_amdgcn_exp2f(m[b] - mn);
+            const float f = corr * fa;
+            m[b] = mn;
+            float sum = 0.f;
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    sc[b][kb][r] = __builtin_amdgcn_exp2f(sc[b][kb][r] - mn);
+                    sum += sc[b][kb][r];
+                }
+            split8(sc[b][0], sc[b][1], ep, ph[b], pl[b]);
+            l[b] = l[b] * corr + sum;
+#pragma unroll
+            for (int db = 0; db < 8; ++db) o[b][db] *= f;
+        }
+        // O^T += V^T P^T, eight blocks of 16 dims, this half's step of 32 keys
 #pragma unroll
         for (int db = 0; db < 8; ++db) {
-            const int e = eb[db >> 1] == aih_operand::kZeroBlock ? 0 : eb[db >> 1];
-            store_operand4(Xt, q_stride, i, (int64_t)h * kHD + 16 * db + 4 * g,
-                           f4{ldexpf(r[db].x, e), ldexpf(r[db].y, e), ldexpf(r[db].z, e), ldexpf(r[db].w, e)});
+            const int at = (16 * db + c) * kRVH + 8 * g + 32 * half;
+            const h8 vh = *reinterpret_cast<const h8 *>(&vsh[at]);
+            const h8 vl = *reinterpret_cast<const h8 *>(&vsh[kHD * kRVH + at]);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) o[b][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[b], o[b][db], 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) o[b][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[b], o[b][db], 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) o[b][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[b], o[b][db], 0, 0, 0);
         }
-        char *const img = reinterpret_cast<char *>(Xt);
-        const int eg = g == 0 ? eb[0] : g == 1 ? eb[1] : g == 2 ? eb[2] : eb[3];
-        reinterpret_cast<int8_t *>(img + aih_operand::block_exp_offset(mpad, q_stride))[i * (q_stride / 32) + 4 * h + g] =
-            (int8_t)eg;
-        if (h == 0 && g == 0) reinterpret_cast<int32_t *>(img + aih_operand::row_exp_offset(mpad, q_stride))[i] = 0;
+        if (it + 2 < n_kt) kv.wave_max(tmax[it & 1], lane, wave);   // tile it + 2's maxima (its loads have landed)
+        ek = ek_next;
+        ev = ev_next;
+        __syncthreads();
+    }
+    // the four lanes of a query hold sums over disjoint keys, all scaled by the same corrections
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        l[b] += __shfl_xor(l[b], 16);
+        l[b] += __shfl_xor(l[b], 32);
+    }
+    // half 1 leaves its unnormalised output and (max, sum) per query in LDS
+    // (64 NB rows of 132 floats, over both images); half 0 merges:
+    //   O = (2^(m0 - M) o0 + 2^(m1 - M) o1) / (2^(m0 - M) l0 + 2^(m1 - M) l1),  M = max(m0, m1)
+    // (a half with no keys has l = 0, o = 0 and m = -FLT_MAX, weight 0)
+    const float u = ldexpf(1.f, -A);
+    static_assert(NB * kQTile * 132 * 4 <= 2 * kImage * 2, "the merge rows fit the images");
+    float *const pub0 = reinterpret_cast<float *>(lds2) + (16 * w + c) * 132;
+    if (half == 1) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            float *const pub = pub0 + b * (kQTile * 132);
+#pragma unroll
+            for (int db = 0; db < 8; ++db) *reinterpret_cast<f4 *>(pub + 16 * db + 4 * g) = o[b][db] * u;
+            if (g == 0) {
+                pub[128] = m[b];
+                pub[129] = l[b];
+            }
+        }
+    }
+    __syncthreads();
+    if (half == 1) return;
+    const int64_t i = i0 + 16 * w + c;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int h = h0 + b;
+        const float *const pub = pub0 + b * (kQTile * 132);
+        f4 r[8];
+        const float m1 = pub[128], l1 = pub[129];
+        const float mm = fmaxf(m[b], m1), a0 = exp2f(m[b] - mm), a1 = exp2f(m1 - mm);
+        const float den = a0 * l[b] + a1 * l1;
+#pragma unroll
+        for (int db = 0; db < 8; ++db)
+            r[db] = (a0 * (o[b][db] * u) + a1 * *reinterpret_cast<const f4 *>(pub + 16 * db + 4 * g)) / den;
+        if (Xt) prefill_operand_rows(Xt, r, i, n_q, q_stride, h, g);
+        else if (i < n_q)
+#pragma unroll
+            for (int db = 0; db < 8; ++db)
+                *reinterpret_cast<f4 *>(O + i * q_stride + (int64_t)h * kHD + 16 * db + 4 * g) = r[db];
     }
 }
 
@@ -1980,6 +2307,33 @@ int aih_add(aih_ctx *ctx, const float *A, const float *B, float *Y, int64_t n)
     return aih_launch_status();
 }
 
+// Whether two heads per workgroup are faster than one: the longest-first
+// schedule of the query tiles' workgroups over the CUs, in key tiles (the
+// longest workgroup, the mean load, and k + 1 workgroups at least as long as
+// the (k cus + 1)-th on some CU), at the measured 3.45 us a tile for two heads
+// and 2.45 us for one.  A position in device memory counts as 0.  Measured at
+// 32 heads, one -> two: 512 queries 28.9 -> 40.3 us (128 workgroups on 256
+// CUs), 1024 59 -> 69, 1500 119 -> 94.  Over 91 shapes (4 to 64 heads, 9 to
+// 2048 queries, positions 0 to 3000) it picks the faster one, or a tie.
+static bool prefill_pairs(const aih_ctx *ctx, int64_t n_q, int32_t n_heads, int32_t n_kv_heads, int32_t start,
+                          int32_t max_len)
+{
+    if (n_heads / n_kv_heads % 2) return false;
+    const int64_t tiles = (n_q + kQTile - 1) / kQTile, cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    auto len = [&](int64_t t) {   // key tiles of query tile t, longest first
+        const int64_t last = std::min<int64_t>(start + std::min<int64_t>((tiles - t) * kQTile, n_q), max_len) - 1;
+        return last < 0 ? 0.0 : (double)(last / kKT + 1);
+    };
+    double sum = 0;
+    for (int64_t t = 0; t < tiles; ++t) sum += len(t);
+    auto load = [&](int64_t heads) {
+        double most = std::max(len(0), sum * (double)heads / (double)cus);
+        for (int64_t k = 1; k * cus < tiles * heads; ++k) most = std::max(most, (double)(k + 1) * len(k * cus / heads));
+        return most;
+    };
+    return 3.45 * load(n_heads / 2) < 2.45 * load(n_heads);
+}
+
 // The tiled (prefill) attention: the output as fp32 rows in O, or, with Xt,
 // as the fp16 operand image of a GEMM over its n_heads * kHD columns.
 static int prefill_attention(aih_ctx *ctx, const float *Q, int64_t ldq, const float *Kc, const float *Vc, float *O,
@@ -1988,8 +2342,12 @@ static int prefill_attention(aih_ctx *ctx, const float *Q, int64_t ldq, const fl
 {
     const int64_t tiles = (n_q + kQTile - 1) / kQTile;
     if (tiles > 65535) return AIH_E_LIMIT;
-    hipLaunchKernelGGL(attn_prefill_kernel, dim3(n_heads, (unsigned)tiles), dim3(512), 0, ctx->stream, Q, ldq, Kc,
-                       Vc, O, n_q, n_heads, n_kv_heads, start, pos, max_len, scale, Xt);
+    if (prefill_pairs(ctx, n_q, n_heads, n_kv_heads, start, max_len))
+        hipLaunchKernelGGL(attn_prefill_group_kernel<2>, dim3(n_heads / 2, (unsigned)tiles), dim3(512), 0, ctx->stream, Q,
+                           ldq, Kc, Vc, O, n_q, n_heads, n_kv_heads, start, pos, max_len, scale, Xt);
+    else
+        hipLaunchKernelGGL(attn_prefill_kernel, dim3(n_heads, (unsigned)tiles), dim3(512), 0, ctx->stream, Q, ldq,
+                           Kc, Vc, O, n_q, n_heads, n_kv_heads, start, pos, max_len, scale, Xt);
     return aih_launch_status();
 }
 

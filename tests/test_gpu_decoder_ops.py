@@ -274,6 +274,30 @@ def test_attention_prefill(device, bufs, n_q, start):
     _attn(device, bufs, n_q, start, 640)
 
 
+# enough query tiles and heads for two heads per workgroup (on a 256-CU
+# device): partial query and key tiles, groups of 8, 2 and 16 heads, a device
+# position; the first rows of each see no key of the second half of a tile
+@pytest.mark.parametrize("n_q,start,nh,nkv,pos", [(800, 0, 64, 8, None), (709, 77, 64, 32, None), (770, 0, 96, 6, 50)])
+def test_attention_prefill_head_pairs(device, bufs, n_q, start, nh, nkv, pos):
+    _attn(device, bufs, n_q, start, start + (pos or 0) + n_q, nh, nkv, pos)
+
+
+def test_attention_prefill_head_pairs_magnitudes(device, bufs):
+    # as below, with V tiles from 1e-6 to 1e6 row by row, and bit for bit
+    # under powers of two
+    nh, nkv, n_q = 64, 8, 800
+    q, K, V = rnd(71, n_q, nh * 128), rnd(72, n_q, nkv * 128), rnd(73, n_q, nkv * 128)
+    V *= (10.0 ** (3 * ((np.arange(n_q) // 64) % 5 - 2))).astype(np.float32)[:, None]
+    q *= (10.0 ** -(np.arange(n_q) % 4)).astype(np.float32)[:, None]
+    o = _run_attn(device, bufs, q, K, V, 0, nh, nkv)
+    ref = ol.attention(q, K, V, list(range(n_q)), nh, nkv, 128)
+    err = np.linalg.norm(o - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert err.max() < 1e-5, err.max()
+    two = np.float32(2.0)
+    assert np.array_equal(_run_attn(device, bufs, q * two ** 40, K * two ** -40, V * two ** -30, 0, nh, nkv),
+                          o * two ** -30)
+
+
 def test_attention_prefill_power_of_two_invariance(device, bufs):
     # the products run on fp16 hi/lo operands with per-row (Q) and per-tile
     # (K, V) powers of two: scaling Q by 2^a, K by 2^-a and V by 2^b changes

@@ -345,6 +345,34 @@ def _operand_image(x, mpad):
     return img
 
 
+def test_attention_operand_of_head_pairs(device):
+    """The same for two heads per workgroup (64 heads, 801 rows on a 256-CU
+    device): the operand is the fp32 output rounded, its exponents zero."""
+    L, h = nat.lib(), device.handle
+    n_q, nh, nkv, qd = 801, 64, 8, 64 * 128
+    rng = np.random.default_rng(17)
+    bufs = [upload(device, rng.standard_normal((n_q, w * 128)).astype(np.float32)) for w in (nh, nkv, nkv)]
+    q, kb, vb = (b.get_pointer() for b in bufs)
+    mpad = (n_q + 31) // 32 * 32
+    raw = np.full(nat.operand_bytes(n_q, qd), 0xFF, np.uint8)   # NaN halves
+    xt, o, sb = upload(device, raw), device.create_buffer(n_q * qd * 4), device.create_buffer(16)
+    try:
+        _check(L.aih_attention(h, q, kb, vb, o.get_pointer(), n_q, nh, nkv, 128, 0, None, n_q, 0.088, sb.get_pointer(),
+                               4), "fp32")
+        _check(L.aih_attention_operand(h, q, qd, kb, vb, xt.get_pointer(), n_q, nh, nkv, 128, 0, None, n_q, 0.088),
+               "operand")
+        nat.check(L.aih_memcpy_d2h(h, raw.ctypes.data, xt.get_pointer(), raw.nbytes), "d2h")
+        img = _operand_image(_read(o, n_q * qd).reshape(n_q, qd), mpad)
+    finally:
+        for b in bufs + [xt, o, sb]:
+            b.dispose()
+    assert np.array_equal(raw[:2 * mpad * qd].view(np.uint16), img.view(np.uint16).reshape(-1))
+    at = 2 * mpad * qd
+    assert not raw[at:at + 4 * mpad].any()
+    blocks = raw[at + 4 * mpad:at + 4 * mpad + mpad * qd // 32].view(np.int8).reshape(mpad, qd // 32)
+    assert np.all(blocks[:n_q] == 0) and np.all(blocks[n_q:] == -128)
+
+
 # (300, 0) has split query tiles (three or more key tiles), (70, 30) a
 # partial last row block, (2, 100) two rows
 @pytest.mark.parametrize("n_q,start", [(300, 0), (70, 30), (2, 100)])
