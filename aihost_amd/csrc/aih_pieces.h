@@ -328,9 +328,38 @@ struct Pair32 {
     }
 };
 
+// Q6_K in 32-weight pieces: half ph of chunk c is quarter Q = 2 * (c % 2) + ph,
+// 32 contiguous bytes of each code array, two scale bytes and one d.  18
+// registers and 6 loads against Pair32's 20 and 8: the 512 x 128 tile, whose
+// accumulators leave few, otherwise spills weights it has just loaded.
+struct G6K32 {
+    struct Raw { u4 ql[2], qh[2]; uint32_t sc, d; };
+    __device__ static void load(const uint8_t *row, int c, int ph, Raw &r)
+    {
+        const uint8_t *b = row + (c >> 2) * 210;
+        const int h = (c & 3) >> 1, Q = 2 * (c & 1) + ph;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            r.ql[t] = ldg<u4>(b + 64 * h + 32 * (Q & 1) + 16 * t);
+            r.qh[t] = ldg<u4>(b + 128 + 32 * h + 16 * t);
+        }
+        r.sc = ldg<uint16_t>(b + 192 + 8 * h + 2 * Q);
+        r.d = ldg<uint16_t>(b + 208);
+    }
+    __device__ static void piece(const Raw &r, int c, int ph, h8 out[4])
+    {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+            G6K::piece_h(G6K::Raw{r.ql[t], r.qh[t], r.sc >> (8 * t), r.d}, c, 2 * ph + t, out[2 * t], out[2 * t + 1]);
+    }
+    __device__ static constexpr int col(int ph, int q) { return Pair32<G6K>::col(ph, q); }
+    __device__ static constexpr int swz(int g) { return Pair32<G6K>::swz(g); }
+};
+
 // The GEMM producers' piece type for format T.
 template <class T> struct Piece32 { typedef Pair32<T> type; };
 template <> struct Piece32<G4K> { typedef G4K32 type; };
+template <> struct Piece32<G6K> { typedef G6K32 type; };
 
 // The 16 weights of piece s of chunk c as two fp16 vectors.
 template <class T>

@@ -491,7 +491,7 @@ qgemm_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
 // super-step s:
 //   - it dequantizes its 8 NB of the 64 NB weight rows (rows 64 i + 8w + lane / 8) for
 //     super-step s+1 into the other LDS buffer, 32 weights per lane
-//     (Piece32), from packed loads PR256 (NB = 2: one) super-steps ahead;
+//     (Piece32), from packed loads PR256 (NB = 2: one) super-steps ahead (Q6_K: see LATE);
 //   - it multiplies super-step s: wave w owns rows 32 MB w .. +32 MB - 1 of
 //     the M tile and all 64 NB columns (2 MB NB 32x32 accumulators: each A fragment
 //     feeds 2 NB, each B fragment MB), A fragments from the tiled X AD 64-k
@@ -519,10 +519,17 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
 {
     static_assert(SC % AD == 0, "A ring depth divides a super-step");
     constexpr int PR = NB == 1 ? PR256 : 1;
+    // Q6_K's 36 registers of packed weights do not fit beside the 512 x 128
+    // accumulators all the way (spilled, they wait for their own loads): they
+    // are loaded in the last chunk before their use, the others a super-step
+    // ahead (Q8_0 loaded late: 3.5% slower).  With the wave index held in a
+    // scalar register (A's addresses too), nothing is spilled in the loop;
+    // 14336 x 4096 x 2048: Q6_K 283 -> 268 us, Q4_K 242 -> 236.
+    constexpr bool LATE = NB > 1 && std::is_same<T, G6K>::value;
     typedef typename Piece32<T>::type Pc;
     typedef typename Pc::Raw Raw;
     __shared__ __align__(16) _Float16 wsh[2][BN * NB][LD2];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t m0 = (int64_t)blockIdx.y * BM2 * MB, n0 = (int64_t)blockIdx.x * (BN * NB);
     const int nch = (int)(K / 64);
     // split z of K (gridDim.z > 1: partial sums into P + z * zs): super-steps
@@ -556,6 +563,7 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
             for (int q = 0; q < 4; ++q)
                 *reinterpret_cast<h8 *>(d + 8 * Pc::swz(8 * pc + Pc::col(ph, q) / 8)) =
                     decltype(tail)::value && c >= nch ? h8{} : o[q];
+            if (NB > 1) __builtin_amdgcn_sched_barrier(0);   // one row's temporaries at a time
         }
     };
 
@@ -626,7 +634,7 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
         auto deq = [&] {
             if (more) {
                 stage(tail, it + 1, buf ^ 1, r);
-                if (reload) gload(it + 1 + PR, r);
+                if (reload && !LATE) gload(it + 1 + PR, r);
             }
             __builtin_amdgcn_sched_barrier(0);
         };
@@ -641,6 +649,7 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
 #pragma unroll
             for (int u = 0; u < 4 * SC; ++u) {
                 if (u + 1 < 4 * SC) bslice(buf, u + 1, bs[(u + 1) & 1]);
+                if (LATE && u == 4 * (SC - 1)) gload(it + (valu_first ? 2 : 1), r);
                 __builtin_amdgcn_sched_barrier(0);
                 AF &a = f[(u >> 2) % AD];
 #pragma unroll
