@@ -239,7 +239,9 @@ struct UQ6K {
 // multiple of 64).  Group g (of 2) contracts block 2t + g of every t < 4, in
 // four windows: in window j lane q holds elements 8j .. 8j + 7 of block
 // 2q + g, so its activations all belong to sub-block t = q.  5..8 columns take
-// two tiles of four columns that share the codes.
+// two tiles of four columns that share the codes.  The activations of a lane's
+// two blocks are one scaling group (64 elements), so that large activations
+// elsewhere in the unit cost them no bits of their hi/lo pairs.
 // On MI355X per call (pieces of 8 bytes -> owned pairs of blocks): Q4_0 14336 x
 // 4096 4 columns 32.9 -> 13.5 us, 8 columns 32.1 -> 18.2, 32000 x 14336 x 8
 // 262 -> 129; Q8_0 14336 x 4096 x 4 30.8 -> 16.5, 4096 x 14336 x 8 35.7 ->
@@ -365,6 +367,10 @@ struct Img {
     float sx[MAXB][NSP];
 };
 
+// Activations that share one power of two S: the T sub-blocks that an MFMA
+// tile contracts, or the two blocks of a lane for the owner formats.
+template <class U, int T> constexpr int kGroup = U::kOwner ? 64 : T * U::SB;
+
 // One round: units ub .. ub+R-1 of the split.  WHOLE: every unit lies inside
 // the row (always for Q4_K/Q6_K; for Q8_0/Q4_0 all but a last partial unit),
 // and the code is straight-line, so that every load of the round is issued
@@ -375,10 +381,10 @@ struct Img {
 // workgroup may still be reading the image.
 template <class U, int T, int CB, int R, bool WHOLE>
 __device__ __forceinline__ void round_of(Rsrc wr, uint32_t rowoff, Rsrc xr, const uint32_t *xo, int ub, int nb,
-                                         int64_t K, int batch, Img<R, T * U::SB, U::SB> &im, bool lead, int tid,
+                                         int64_t K, int batch, Img<R, kGroup<U, T>, U::SB> &im, bool lead, int tid,
                                          int q, const int *xrow, float *out)
 {
-    constexpr int SB = U::SB, G = T * SB, WPG = G / 32, NGU = UNIT / G, CPC = 32 * R;
+    constexpr int SB = U::SB, G = kGroup<U, T>, WPG = G / 32, NGU = UNIT / G, CPC = 32 * R;
     const uint32_t xso = (uint32_t)ub * (UNIT * 4);
     f4 xv[R][2];
 #pragma unroll
@@ -460,7 +466,7 @@ __device__ __forceinline__ void round_of(Rsrc wr, uint32_t rowoff, Rsrc xr, cons
             for (int g = 0; g < 2; ++g) k[g] = pair_scale(rw[u], q, g, U::kScale);
 #pragma unroll
             for (int b = 0; b < CB; ++b) {
-                fv[b] = im.f[b][u * NGU + q / 2];   // both blocks of the lane in one staged group
+                fv[b] = im.f[b][u * NGU + q];   // the lane's two blocks are group q of the unit
 #pragma unroll
                 for (int g = 0; g < 2; ++g) sv[b][g] = im.sx[b][u * 8 + 2 * q + g];
             }
@@ -549,7 +555,8 @@ qmv_split_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes, cons
                  int64_t ldx, int batch, int ntiles, int per, float *__restrict__ P, int64_t np,
                  float *__restrict__ Y, int64_t ldy)
 {
-    constexpr int SB = U::SB, G = T * SB, WPG = G / 32;
+    constexpr int SB = U::SB, G = kGroup<U, T>;
+    constexpr int WPG = U::kOwner ? CB / 4 : G / 32;   // A fragment rows of a lane: column halves, or windows
     __shared__ __align__(16) Img<UPW, G, SB> im;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -585,7 +592,7 @@ qmv_split_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes, cons
     // in window wg of a group when lane q's 8 elements lie in sub-block i % T.
     // Elsewhere the lane reads the zero row.
     int xrow[WPG];
-    static_assert(!U::kOwner || (T == 4 && WPG == 4 && CB <= 8), "owner formats: four sub-blocks per tile");
+    static_assert(!U::kOwner || (T == 4 && SB == 32 && CB <= 8), "owner formats: four blocks per tile");
 #pragma unroll
     for (int wg = 0; wg < WPG; ++wg) {
         const int b = U::kOwner ? n16 % 4 + 4 * wg : n16 / T, t = U::kOwner ? n16 / 4 : n16 % T;

@@ -3,8 +3,8 @@
 The reference multiplies fp32 activations by fp32 weights
 (ComputeShaders.cs:93-129, TransformerBase.cs:454-456): any finite fp32 row is
 a valid input.  The batch-1/2 matvec holds x as 22-bit fixed point per
-64-element unit and the batch-3..8 matvec as fp16 hi/lo pairs per 32-element
-group, each with a power of two from the unit's or group's maximum; the GEMM
+64-element unit and the batch-3..8 matvec as fp16 hi/lo pairs per group of 32
+to 128 elements (64 for Q8_0 and Q4_0), each with a power of two from the unit's or group's maximum; the GEMM
 rounds x to fp16 with a power of two per row (a row above 65504 or far below 1
 keeps its 11 significant bits).  Inputs here:
 
@@ -86,6 +86,24 @@ def test_matvec_activation_range(device, orc, qtype, n, k, batch, kind):
     nrm, mx = check_rows(y, ref, 2e-5, "type %d %dx%d b%d %s" % (qtype, n, k, batch, kind))
     o_nrm = max(np.linalg.norm(ref[b] - r64[b]) / np.linalg.norm(r64[b]) for b in range(batch))
     print("type=%d b%d %s: normwise %.3g max %.3g (oracle vs fp64 %.3g)" % (qtype, batch, kind, nrm, mx, o_nrm))
+
+
+# Runs of 64 large activations that meet zero-scale weight blocks, between runs
+# of 64 small ones that make up the whole result: the small ones keep their
+# bits only if no large one shares their power of two.
+@pytest.mark.parametrize("ratio", [2.0 ** -20, 2.0 ** -28])
+@pytest.mark.parametrize("batch", [3, 4, 5, 8])
+@pytest.mark.parametrize("qtype", [nat.Q8_0, nat.Q4_0])
+def test_matvec_small_runs_beside_large_ones(device, orc, qtype, batch, ratio):
+    n, k = 130, 2112                                    # a partial last unit
+    w = np.frombuffer(synth_weight(qtype, n, k, seed=n + batch), np.uint8).reshape(n, k // 32, -1).copy()
+    run = np.arange(k) // 64
+    x = np.random.default_rng(batch).standard_normal((batch, k)).astype(np.float32)
+    x[:, run % 2 == 1] *= np.float32(ratio)
+    w[:, run[::32] % 2 == 0, :2] = 0                    # fp16 scale
+    w = w.reshape(-1)
+    y = qmatvec(device, qtype, w, n, k, x)[:, :n]
+    check_rows(y, orc.matvec(qtype, w, n, k, x), 2e-5, "type %d b%d" % (qtype, batch))
 
 
 @pytest.mark.parametrize("kind", KINDS)
