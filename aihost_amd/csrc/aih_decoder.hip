@@ -1691,12 +1691,20 @@ attn_prefill_group_kernel(const float *__restrict__ Q, int64_t ldq, const float 
     const int64_t qpos = p0 + min<int64_t>(i0 + 16 * w + c, n_q - 1);   // last key the query attends to
     const float sl = scale * 1.44269504088896341f;                       // scale log2(e)
     float m[NB], l[NB];
-    int A = 1 << 20;   // O accumulators hold 2^A O (lowered by the first tile)
+    // The accumulators of query c hold 2^A O and stay below `top` in magnitude.
+    // Both halves see every tile, so a tile of large V must not take bits from
+    // the rest of the row: A follows each tile up again (P'' = P 2^(A - ev) at
+    // its full 2^15), short only of lifting `top` past 2^120, where what the
+    // accumulators hold outweighs the tile.
+    int A[NB];
+    float top[NB];
     f4 o[NB][8];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         m[b] = -FLT_MAX;   // finite: a half whose keys so far are all masked keeps weight 0
         l[b] = 0.f;
+        A[b] = 1 << 20;   // set by the first tile
+        top[b] = 0.f;
 #pragma unroll
         for (int db = 0; db < 8; ++db) o[b][db] = f4{0.f, 0.f, 0.f, 0.f};
     }
@@ -1754,10 +1762,6 @@ attn_prefill_group_kernel(const float *__restrict__ Q, int64_t ldq, const float 
         // multiplier), causal mask, online softmax of query c in base 2
         // (the half's keys past lim are masked)
         const int lim = (int)max<int64_t>(min<int64_t>(qpos - j0, kKT), -1) - 32 * half;
-        const int An = min(A, ev + 15);
-        const float fa = ldexpf(1.f, max(An - A, -160));
-        A = An;
-        const int ep = An - ev;   // P'' = P 2^(A - ev) <= 2^15
         h8 ph[NB], pl[NB];
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
@@ -1773,7 +1777,11 @@ attn_prefill_group_kernel(const float *__restrict__ Q, int64_t ldq, const float 
                 }
             mx = xor_lanes_max(mx);
             const float mn = fmaxf(m[b], mx), corr = __builtin_amdgcn_exp2f(m[b] - mn);
-            const float f = corr * fa;
+            const float t = __builtin_fmaf(top[b], corr, FLT_MIN);
+            const int dA = min(ev + 15 - A[b], 120 - __builtin_amdgcn_frexp_expf(t));
+            const float f = ldexpf(corr, dA);
+            top[b] = ldexpf(t, dA) + 0x1p37f;   // 32 keys of |P''| <= 2^15, |V''| <= 2^16
+            A[b] += dA;
             m[b] = mn;
             float sum = 0.f;
 #pragma unroll
@@ -1783,7 +1791,7 @@ attn_prefill_group_kernel(const float *__restrict__ Q, int64_t ldq, const float 
                     sc[b][kb][r] = __builtin_amdgcn_exp2f(sc[b][kb][r] - mn);
                     sum += sc[b][kb][r];
                 }
-            split8(sc[b][0], sc[b][1], ep, ph[b], pl[b]);
+            split8(sc[b][0], sc[b][1], A[b] - ev, ph[b], pl[b]);
             l[b] = l[b] * corr + sum;
 #pragma unroll
             for (int db = 0; db < 8; ++db) o[b][db] *= f;
@@ -1816,15 +1824,20 @@ attn_prefill_group_kernel(const float *__restrict__ Q, int64_t ldq, const float 
     // (64 NB rows of 132 floats, over both images); half 0 merges:
     //   O = (2^(m0 - M) o0 + 2^(m1 - M) o1) / (2^(m0 - M) l0 + 2^(m1 - M) l1),  M = max(m0, m1)
     // (a half with no keys has l = 0, o = 0 and m = -FLT_MAX, weight 0)
-    const float u = ldexpf(1.f, -A);
     static_assert(NB * kQTile * 132 * 4 <= 2 * kImage * 2, "the merge rows fit the images");
     float *const pub0 = reinterpret_cast<float *>(lds2) + (16 * w + c) * 132;
+    auto unscaled = [&](int b, int db) {   // 2^-A o
+        f4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = ldexpf(o[b][db][j], -A[b]);
+        return v;
+    };
     if (half == 1) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             float *const pub = pub0 + b * (kQTile * 132);
 #pragma unroll
-            for (int db = 0; db < 8; ++db) *reinterpret_cast<f4 *>(pub + 16 * db + 4 * g) = o[b][db] * u;
+            for (int db = 0; db < 8; ++db) *reinterpret_cast<f4 *>(pub + 16 * db + 4 * g) = unscaled(b, db);
             if (g == 0) {
                 pub[128] = m[b];
                 pub[129] = l[b];
@@ -1844,7 +1857,7 @@ attn_prefill_group_kernel(const float *__restrict__ Q, int64_t ldq, const float 
         const float den = a0 * l[b] + a1 * l1;
 #pragma unroll
         for (int db = 0; db < 8; ++db)
-            r[db] = (a0 * (o[b][db] * u) + a1 * *reinterpret_cast<const f4 *>(pub + 16 * db + 4 * g)) / den;
+            r[db] = (a0 * unscaled(b, db) + a1 * *reinterpret_cast<const f4 *>(pub + 16 * db + 4 * g)) / den;
         if (Xt) prefill_operand_rows(Xt, r, i, n_q, q_stride, h, g);
         else if (i < n_q)
 #pragma unroll

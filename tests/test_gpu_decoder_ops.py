@@ -298,6 +298,24 @@ def test_attention_prefill_head_pairs_magnitudes(device, bufs):
                           o * two ** -30)
 
 
+@pytest.mark.parametrize("big", [2.0 ** 30, 2.0 ** 40, 2.0 ** 90])
+def test_attention_prefill_head_pairs_large_values_of_small_weight(device, bufs, big):
+    # the first 64 keys hold V rows of size `big` at a weight of about 2^-101:
+    # they must not take bits from the keys that make up the result (rows from
+    # 64 on, 1e-5 as above)
+    nh, nkv, n_q = 64, 8, 800
+    q, K, V = rnd(81, n_q, nh * 128), rnd(82, n_q, nkv * 128), rnd(83, n_q, nkv * 128)
+    q[:, ::128] = 8.0
+    K[:, ::128] = 0.0
+    K[:64, ::128] = -99.0            # scores lower by 8 * 99 / sqrt(128) = 70 = 101 ln 2
+    V[:64] *= np.float32(big)
+    o = _run_attn(device, bufs, q, K, V, 0, nh, nkv)
+    ref = ol.attention(q, K, V, list(range(n_q)), nh, nkv, 128)
+    d = np.linalg.norm((o - ref)[64:].astype(np.float64), axis=1)
+    worst = float(np.max(d / np.linalg.norm(ref[64:].astype(np.float64), axis=1)))
+    assert worst < 1e-5, worst
+
+
 def test_attention_prefill_power_of_two_invariance(device, bufs):
     # the products run on fp16 hi/lo operands with per-row (Q) and per-tile
     # (K, V) powers of two: scaling Q by 2^a, K by 2^-a and V by 2^b changes
