@@ -466,11 +466,11 @@ qgemm_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
         }
     }
 
-    undo_row_exp(acc0, acc1, ev, E, mb * 32, lane);
-    if (P) {   // a split's partial sums (the summing pass applies the epilogue)
+    if (P) {   // a split's partial sums (the summing pass undoes the exponents and applies the epilogue)
         store_tile(acc0, acc1, lane, m0 + 32 * wave, n0, M, N, P + (int64_t)blockIdx.z * zs, false);
         return;
     }
+    undo_row_exp(acc0, acc1, ev, E, mb * 32, lane);
     if (epi == kEpiSiluOperand) {
         // the tile buffer of super-step nss: nothing reads or writes it any more
         silu_pairs_operand(acc0, acc1, lane, m0 + 32 * wave, n0, M, N,
@@ -703,12 +703,14 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
         if (it < nss) body(std::true_type{}, it, ring[(j + 1) % PR], it + 1 < nss, it + 1 + PR < nss);
     }
 
+    if (!P) {   // the summing pass undoes a split's
 #pragma unroll
-    for (int j = 0; j < MB; ++j) {
-        int64_t mb = (m0 + 32 * (MB * wave + j)) / 32;
-        mb = mb < mblocks ? mb : mblocks - 1;
+        for (int j = 0; j < MB; ++j) {
+            int64_t mb = (m0 + 32 * (MB * wave + j)) / 32;
+            mb = mb < mblocks ? mb : mblocks - 1;
 #pragma unroll
-        for (int i = 0; i < NB; ++i) undo_row_exp(acc[j][2 * i], acc[j][2 * i + 1], ev[j], E, mb * 32, lane);
+            for (int i = 0; i < NB; ++i) undo_row_exp(acc[j][2 * i], acc[j][2 * i + 1], ev[j], E, mb * 32, lane);
+        }
     }
     // every 32 x 64 block b = j NB + i (row fragment j, column pair i) of the
     // wave, unrolled by hand: the epilogues are too large for the pragma
@@ -751,6 +753,14 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
     });
 }
 
+// Partial sums keep their row's power of two (aih_operand.h): those of a row of
+// large values may exceed fp32 where their sum does not.  The summing passes
+// undo it, row m's being E[m].
+__device__ __forceinline__ f4 undo_row_exp4(f4 s, int e)
+{
+    return e == 0 ? s : f4{ldexpf(s.x, -e), ldexpf(s.y, -e), ldexpf(s.z, -e), ldexpf(s.w, -e)};
+}
+
 // The sum of the splits' partial sums p[0], p[zs], ... (in that order).
 __device__ __forceinline__ f4 split_sum4(const float *__restrict__ p, int S, int64_t zs)
 {
@@ -771,12 +781,20 @@ __device__ __forceinline__ f4 split_sum4(const float *__restrict__ p, int S, int
 // added into Y (Y + sum, the order of the accumulate epilogue) when
 // `accumulate`.  Splits are zs floats apart (a multiple of 4, at least MN).
 // Four elements per thread (16-byte accesses of Y when it is 16-byte aligned).
+// MN fits 32 bits: a split product has fewer tiles than the device has CUs.
 template <bool VEC>
 __global__ void __launch_bounds__(256)
-split_k_sum_kernel(const float *__restrict__ P, int S, int64_t MN, int64_t zs, float *__restrict__ Y, int accumulate)
+split_k_sum_kernel(const float *__restrict__ P, int S, int64_t MN, uint32_t N, int64_t zs,
+                   const int32_t *__restrict__ E, float *__restrict__ Y, int accumulate)
 {
     for (int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x); i < MN; i += 4 * (int64_t)gridDim.x * 256) {
-        const f4 s = split_sum4(P + i, S, zs);
+        f4 s = split_sum4(P + i, S, zs);
+        if (N % 4 == 0) {
+            s = undo_row_exp4(s, E[(uint32_t)i / N]);
+        } else {   // the four elements may lie in several rows (past the end: the last row's)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] = ldexpf(s[j], -E[(uint32_t)min<int64_t>(i + j, MN - 1) / N]);
+        }
         if (VEC && i + 4 <= MN) {
             f4 *y = reinterpret_cast<f4 *>(Y + i);
             *y = accumulate ? *y + s : s;
@@ -789,16 +807,16 @@ split_k_sum_kernel(const float *__restrict__ P, int S, int64_t MN, int64_t zs, f
 }
 
 // The same sum with the Q|K|V epilogue: what rope_qkv_block stores, two pairs
-// (four columns) per thread.  N and the head boundaries are multiples of 32.
+// (four columns) per thread, one row (of at most 256) per blockIdx.y.  N and the
+// head boundaries are multiples of 32.
 __global__ void __launch_bounds__(256)
-split_k_rope_kernel(const float *__restrict__ P, int S, int64_t M, int64_t N, int64_t zs, float *__restrict__ Y,
-                    const aih_rope_qkv_args ra)
+split_k_rope_kernel(const float *__restrict__ P, int S, int64_t N, int64_t zs,
+                    const int32_t *__restrict__ E, float *__restrict__ Y, const aih_rope_qkv_args ra)
 {
 #pragma clang fp contract(off)
-    const int64_t t = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
-    if (t >= M * N) return;
-    const int64_t m = t / N, n = t % N;
-    const f4 x = split_sum4(P + t, S, zs);
+    const int64_t m = blockIdx.y, n = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x), t = m * N + n;
+    if (n >= N) return;
+    const f4 x = undo_row_exp4(split_sum4(P + t, S, zs), E[m]);
     const int64_t p = (int64_t)ra.start + (ra.pos ? *ra.pos : 0) + m;
     const bool in_table = p >= 0 && p < ra.table_rows, in_cache = in_table && p < ra.cache_rows;
     const int kind = n < ra.qd ? 0 : n < (int64_t)ra.qd + ra.kvd ? 1 : 2;
@@ -822,7 +840,8 @@ split_k_rope_kernel(const float *__restrict__ P, int S, int64_t M, int64_t N, in
 // the image); the four threads of a 32-output block share its exponent.
 // N is a multiple of 64; rows M .. mpad - 1 are zero.
 __global__ void __launch_bounds__(256)
-split_k_silu_kernel(const float *__restrict__ P, int S, int64_t M, int64_t N, int64_t zs, _Float16 *__restrict__ out)
+split_k_silu_kernel(const float *__restrict__ P, int S, int64_t M, int64_t N, int64_t zs,
+                    const int32_t *__restrict__ E, _Float16 *__restrict__ out)
 {
     const int64_t mpad = aih_operand::mpad_of(M), kd = N / 2, per_row = N / 16;
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -830,9 +849,10 @@ split_k_silu_kernel(const float *__restrict__ P, int S, int64_t M, int64_t N, in
     const bool live = m < M;   // whole groups of four threads alike (per_row is a multiple of 4)
     float v[8] = {};
     if (live) {
+        const int e = E[m];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const f4 x = split_sum4(P + m * N + 16 * c + 4 * q, S, zs);
+            const f4 x = undo_row_exp4(split_sum4(P + m * N + 16 * c + 4 * q, S, zs), e);
             v[2 * q] = (x.x * (1.0f / (1.0f + expf(-x.x)))) * x.y;
             v[2 * q + 1] = (x.z * (1.0f / (1.0f + expf(-x.z)))) * x.w;
         }
@@ -999,20 +1019,21 @@ GemmPlan plan_gemm(int64_t cu_count, int64_t N, int64_t K, int64_t M, int epi, b
     return p;
 }
 
-// The summing pass of a split product, with its epilogue.
-int launch_split_sum(aih_ctx *ctx, const float *P, const GemmPlan &p, int64_t M, int64_t N, float *Y, int epi,
-                     const aih_rope_qkv_args &ra)
+// The summing pass of a split product, with its epilogue; E: the operand's row
+// exponents.
+int launch_split_sum(aih_ctx *ctx, const float *P, const GemmPlan &p, int64_t M, int64_t N, const int32_t *E, float *Y,
+                     int epi, const aih_rope_qkv_args &ra)
 {
     const int64_t zs = split_stride(M, N);
     if (epi == kEpiRopeQKV) {
-        hipLaunchKernelGGL(split_k_rope_kernel, dim3((unsigned)((M * N / 4 + 255) / 256)), dim3(256), 0, ctx->stream, P,
-                           p.splits, M, N, zs, Y, ra);
+        hipLaunchKernelGGL(split_k_rope_kernel, dim3((unsigned)((N / 4 + 255) / 256), (unsigned)M), dim3(256), 0, ctx->stream, P,
+                           p.splits, N, zs, E, Y, ra);
         return aih_launch_status();
     }
     if (epi == kEpiSiluOperand) {
         const int64_t threads = aih_operand::mpad_of(M) * (N / 16);
         hipLaunchKernelGGL(split_k_silu_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, ctx->stream, P,
-                           p.splits, M, N, zs, reinterpret_cast<_Float16 *>(Y));
+                           p.splits, M, N, zs, E, reinterpret_cast<_Float16 *>(Y));
         return aih_launch_status();
     }
     const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
@@ -1020,9 +1041,11 @@ int launch_split_sum(aih_ctx *ctx, const float *P, const GemmPlan &p, int64_t M,
     const dim3 grid((unsigned)std::min<int64_t>(groups, 8 * cus));
     const int add = epi == kEpiAccumulate ? 1 : 0;
     if (reinterpret_cast<uintptr_t>(Y) % 16 == 0)
-        hipLaunchKernelGGL(split_k_sum_kernel<true>, grid, dim3(256), 0, ctx->stream, P, p.splits, M * N, zs, Y, add);
+        hipLaunchKernelGGL(split_k_sum_kernel<true>, grid, dim3(256), 0, ctx->stream, P, p.splits, M * N, (uint32_t)N, zs, E,
+                           Y, add);
     else
-        hipLaunchKernelGGL(split_k_sum_kernel<false>, grid, dim3(256), 0, ctx->stream, P, p.splits, M * N, zs, Y, add);
+        hipLaunchKernelGGL(split_k_sum_kernel<false>, grid, dim3(256), 0, ctx->stream, P, p.splits, M * N, (uint32_t)N, zs, E,
+                           Y, add);
     return aih_launch_status();
 }
 
@@ -1069,7 +1092,10 @@ int launch(aih_ctx *ctx, const uint8_t *W, int64_t N, int64_t K, int64_t row_byt
         hipLaunchKernelGGL((qgemm_kernel<T>), dim3((unsigned)gx, (unsigned)gy, gz), dim3(64 * (4 + GRing<T>::NP)), 0, ctx->stream,
                            W, N, K, row_bytes, Xh, M, Y, epi, P, zs, p.ssper, ra);
     const int rc = aih_launch_status();
-    return rc || p.splits == 1 ? rc : launch_split_sum(ctx, P, p, M, N, Y, epi, ra);
+    if (rc || p.splits == 1) return rc;
+    const int32_t *const E = reinterpret_cast<const int32_t *>(
+        reinterpret_cast<const char *>(Xh) + aih_operand::row_exp_offset(aih_operand::mpad_of(M), K));
+    return launch_split_sum(ctx, P, p, M, N, E, Y, epi, ra);
 }
 
 }  // namespace

@@ -29,6 +29,7 @@ import numpy as np
 import pytest
 
 from aihost_amd import _native as nat
+from aihost_amd import compute as C
 from gpu_util import qgemm, qmatvec, synth_weight, upload
 
 pytestmark = pytest.mark.gpu
@@ -124,12 +125,32 @@ def test_gemm_activation_range(device, orc, qtype, n, k, m, kind):
 
 def test_gemm_split_k_rows_scaled(device, orc):
     """The down-projection shape, whose GEMM splits K over workgroups on a
-    256-CU device: each split's partial sums carry the row exponents undone."""
+    256-CU device: the row exponents are undone in the sum of the splits."""
     n, k, m = 4096, 14336, 512
     w = synth_weight(nat.Q4_K, n, k, seed=3)
     x = activations("rows_1e5_1e-6", m, k, seed=9)
     y = qgemm(device, nat.Q4_K, w, n, k, x)
     check_rows(y, orc.matvec(nat.Q4_K, w, n, k, x, nthreads=16), 1e-3, "split K")
+
+
+# Rows near the end of fp32 whose first half of K is positive and second half
+# negative: the sums over a split of K exceed fp32, their total does not.  A
+# power of two changes no bit of the product, so it equals the one of rows 2^-64
+# as large; odd N (a row's end inside a thread's four outputs) and both widths
+# of split product.
+@pytest.mark.parametrize("n,m", [(256, 33), (255, 130), (4096, 512)])
+def test_gemm_split_sums_past_fp32(device, n, m):
+    k = 14336
+    if device.info().compute_units == 256:
+        assert nat.qgemm_plan(device.handle, n, k, m)[1] > 1
+    rng = np.random.default_rng(n)
+    w = C.quantize(nat.Q8_0, np.abs(C.fill_normal(4, n * k, 0.0, 0.02)), n, k)
+    x = (1.0 + 0.125 * rng.standard_normal((m, k))).astype(np.float32)
+    x[:, k // 2:] *= -1.0
+    x *= np.exp2(rng.integers(120, 125, m)).astype(np.float32)[:, None]
+    small = qgemm(device, nat.Q8_0, w, n, k, x * np.float32(2.0 ** -64))
+    assert np.abs(small).max() < 2.0 ** 63
+    assert np.array_equal(qgemm(device, nat.Q8_0, w, n, k, x), small * np.float32(2.0 ** 64))
 
 
 # ---------------------------------------------------------------- operand images

@@ -124,13 +124,13 @@ def test_qgemm_fused_equals_separate_operators(device, qtype, n, k, m):
 # takes the 256-row tiles for gate|up on a 256-CU device, (512, 128, 40) the
 # 128-row tiles
 @pytest.mark.parametrize("d,f,m,qt_down", [(512, 128, 40, nat.Q8_0), (1024, 3072, 300, nat.Q4_K)])
-def test_silu_pairs_operand_chain_equals_separate_operators(device, d, f, m, qt_down):
+def test_silu_pairs_operand_chain_equals_separate_operators(device, d, f, m, qt_down, norm=1.0):
     L, h = nat.lib(), device.handle
     rng = np.random.default_rng(d + f + m)
     w_gu = synth_weight(nat.Q4_K, 2 * f, d, seed=d)
     w_dn = synth_weight(qt_down, d, f, seed=f)
     x = rng.standard_normal((m, d)).astype(np.float32)
-    nw = (1.0 + 0.1 * rng.standard_normal(d)).astype(np.float32)
+    nw = (norm * (1.0 + 0.1 * rng.standard_normal(d))).astype(np.float32)
     y0 = rng.standard_normal((m, d)).astype(np.float32)
     bufs = [upload(device, a) for a in (w_gu, w_dn, x, nw)]
     wgu, wdn, xb, nb = bufs
@@ -163,6 +163,8 @@ def test_silu_pairs_operand_chain_with_split_k(device, m):
     if device.info().compute_units == 256:
         assert nat.qgemm_plan(device.handle, 640, 4096, m)[1] > 1
     test_silu_pairs_operand_chain_equals_separate_operators(device, 4096, 320, m, nat.Q8_0)
+    # rows past fp16: the summing pass undoes their power of two
+    test_silu_pairs_operand_chain_equals_separate_operators(device, 4096, 320, m, nat.Q8_0, norm=1e6)
 
 
 def test_qgemm_fused_argument_errors(device):
@@ -202,7 +204,7 @@ QKV_CASES = [(4, 2, 256, 40, 0, None, 64, 64, nat.PRE_RMSNORM, nat.Q4_K),
 
 
 @pytest.mark.parametrize("nh,nkv,k,m,start,dpos,trows,crows,pre,qtype", QKV_CASES)
-def test_qkv_rope_gemm_equals_gemm_then_rope(device, nh, nkv, k, m, start, dpos, trows, crows, pre, qtype):
+def test_qkv_rope_gemm_equals_gemm_then_rope(device, nh, nkv, k, m, start, dpos, trows, crows, pre, qtype, norm=1.0):
     """aih_qgemm_qkv_rope against aih_qgemm_fused (store) + aih_rope_qkv: the
     rotated queries and both caches bit for bit; the key and value columns of
     its Q are left as they were."""
@@ -213,7 +215,7 @@ def test_qkv_rope_gemm_equals_gemm_then_rope(device, nh, nkv, k, m, start, dpos,
     rng = np.random.default_rng(nh + k + m)
     w = synth_weight(qtype, n, k, seed=k + 1)
     x = rng.standard_normal((m, k)).astype(np.float32)
-    nw = (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    nw = (norm * (1.0 + 0.1 * rng.standard_normal(k))).astype(np.float32)
     cache0 = rng.standard_normal((crows, kvd)).astype(np.float32)
     q0 = np.full((m, n), 7.0, np.float32)
     bufs = [upload(device, a) for a in (w, x, nw, cache0, cache0, cache0, cache0, q0, q0)]
@@ -258,6 +260,8 @@ def test_qkv_rope_gemm_with_split_k(device, m, start, dpos, trows, crows):
     if device.info().compute_units == 256:
         assert nat.qgemm_plan(device.handle, 1024, 4096, m)[1] > 1
     test_qkv_rope_gemm_equals_gemm_then_rope(device, 4, 2, 4096, m, start, dpos, trows, crows, nat.PRE_RMSNORM, nat.Q4_K)
+    test_qkv_rope_gemm_equals_gemm_then_rope(device, 4, 2, 4096, m, start, dpos, trows, crows, nat.PRE_RMSNORM, nat.Q4_K,
+                                             norm=1e6)
 
 
 # both fused epilogues over the 512 x 128 tiles (N = 6144 and 8064)
