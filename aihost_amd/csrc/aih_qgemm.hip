@@ -317,7 +317,7 @@ qgemm_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
     constexpr int RPW = BN / GRing<T>::NP;   // weight rows per producer wave
     constexpr int NR = P32 ? RPW / 8 : RPW / 4;   // row groups per producer wave
     __shared__ __align__(16) _Float16 wsh[2][BN][LD2];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
     const int nch = (int)(K / 64);
     // split z of K (gridDim.z > 1: partial sums into P + z * zs): super-steps
@@ -511,6 +511,16 @@ qgemm_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
 constexpr int BM2 = 256;
 constexpr int PR256 = 2;
 
+// This lane's index, computed again: the epilogue of the 512 x 128 tile would
+// otherwise hold it, and what is derived from it, in registers that the loop
+// then spills.
+__device__ __forceinline__ int lane_id()
+{
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
+
 template <class T, int MB, int NB, int AD>
 __global__ void __launch_bounds__(512)
 qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
@@ -551,6 +561,11 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
 #pragma unroll
         for (int i = 0; i < NB; ++i) Pc::load(wrow[i], c, ph, r[i]);
     };
+    // LDS positions of this lane in one index each (swz permutes the bits of a
+    // granule's index and leaves bit 0 in place): where it stores piece 0, and
+    // where it reads granule 2u + (lane / 32)
+    const int wat = (8 * wave + rl) * LD2 + 8 * Pc::swz(8 * pc + Pc::col(ph, 0) / 8);
+    const int rat = (lane & 31) * LD2 + 8 * (lane >> 5);
     // chunks past K exist only in a last, partial super-step, staged as zeros
     auto stage = [&](auto tail, int ss, int buf, const Raw *r) {
         const int c = (ss0 + ss) * SC + pc;
@@ -558,10 +573,10 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
         for (int i = 0; i < NB; ++i) {
             h8 o[4];
             Pc::piece(r[i], c, ph, o);
-            _Float16 *d = &wsh[buf][64 * i + 8 * wave + rl][0];
+            _Float16 *d = &wsh[buf][64 * i][0] + wat;
 #pragma unroll
             for (int q = 0; q < 4; ++q)
-                *reinterpret_cast<h8 *>(d + 8 * Pc::swz(8 * pc + Pc::col(ph, q) / 8)) =
+                *reinterpret_cast<h8 *>(d + 8 * Pc::swz(Pc::col(0, q) / 8)) =
                     decltype(tail)::value && c >= nch ? h8{} : o[q];
             if (NB > 1) __builtin_amdgcn_sched_barrier(0);   // one row's temporaries at a time
         }
@@ -578,7 +593,7 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
         int64_t mb = (m0 + 32 * (MB * wave + j)) / 32;
         mb = mb < mblocks ? mb : mblocks - 1;
         xa[j] = Xt + (mb * kc * 64 + lane) * 8;
-        ev[j] = E[mb * 32 + (lane & 31)];
+        if (NB == 1) ev[j] = E[mb * 32 + (lane & 31)];
     }
     struct AF { h8 a[MB][4]; };
     auto aload = [&](int kb, AF &f) {
@@ -614,7 +629,7 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
     auto bslice = [&](int buf, int u, BS &b) {
 #pragma unroll
         for (int i = 0; i < 2 * NB; ++i)
-            b.b[i] = *reinterpret_cast<const h8 *>(&wsh[buf][32 * i + fr][8 * Pc::swz(2 * u + fk / 8)]);
+            b.b[i] = *reinterpret_cast<const h8 *>(&wsh[buf][32 * i][8 * Pc::swz(2 * u)] + rat);
     };
 
     // Iteration it: products of super-step it from buffer it & 1, and, if
@@ -703,13 +718,15 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
         if (it < nss) body(std::true_type{}, it, ring[(j + 1) % PR], it + 1 < nss, it + 1 + PR < nss);
     }
 
+    const int el = lane_id();
     if (!P) {   // the summing pass undoes a split's
 #pragma unroll
         for (int j = 0; j < MB; ++j) {
             int64_t mb = (m0 + 32 * (MB * wave + j)) / 32;
             mb = mb < mblocks ? mb : mblocks - 1;
+            if (NB > 1) ev[j] = E[mb * 32 + (el & 31)];
 #pragma unroll
-            for (int i = 0; i < NB; ++i) undo_row_exp(acc[j][2 * i], acc[j][2 * i + 1], ev[j], E, mb * 32, lane);
+            for (int i = 0; i < NB; ++i) undo_row_exp(acc[j][2 * i], acc[j][2 * i + 1], ev[j], E, mb * 32, el);
         }
     }
     // every 32 x 64 block b = j NB + i (row fragment j, column pair i) of the
@@ -727,7 +744,7 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
         each([&](auto bc) {
             constexpr int b = decltype(bc)::value;
             if (NB == 1 || n0 + 64 * (b % NB) < N)
-                silu_pairs_operand(acc[b / NB][2 * (b % NB)], acc[b / NB][2 * (b % NB) + 1], lane,
+                silu_pairs_operand(acc[b / NB][2 * (b % NB)], acc[b / NB][2 * (b % NB) + 1], el,
                                    m0 + 32 * (MB * wave + b / NB), n0 + 64 * (b % NB), M, N,
                                    reinterpret_cast<float *>(&wsh[0][0][0]) + wave * 32 * 36,
                                    reinterpret_cast<_Float16 *>(Y));
@@ -740,7 +757,7 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
     if (epi == kEpiRopeQKV) {   // never split here (the plan splits this epilogue over 128-row tiles only)
         each([&](auto bc) {
             constexpr int j = decltype(bc)::value / NB, i = decltype(bc)::value % NB;
-            rope_qkv_tile(acc[j][2 * i], acc[j][2 * i + 1], lane, m0 + 32 * (MB * wave + j), n0 + 64 * i, M, N, Y, ra);
+            rope_qkv_tile(acc[j][2 * i], acc[j][2 * i + 1], el, m0 + 32 * (MB * wave + j), n0 + 64 * i, M, N, Y, ra);
         });
         return;
     }
@@ -748,7 +765,7 @@ qgemm256_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
     float *const Pz = P ? P + (int64_t)blockIdx.z * zs : nullptr;
     each([&](auto bc) {
         constexpr int j = decltype(bc)::value / NB, i = decltype(bc)::value % NB;
-        store_tile(acc[j][2 * i], acc[j][2 * i + 1], lane, m0 + 32 * (MB * wave + j), n0 + 64 * i, M, N, Pz ? Pz : Y,
+        store_tile(acc[j][2 * i], acc[j][2 * i + 1], el, m0 + 32 * (MB * wave + j), n0 + 64 * i, M, N, Pz ? Pz : Y,
                    !Pz && epi == kEpiAccumulate);
     });
 }
