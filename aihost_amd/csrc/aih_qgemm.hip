@@ -805,9 +805,10 @@ split_k_sum_kernel(const float *__restrict__ P, int S, int64_t MN, uint32_t N, i
                    const int32_t *__restrict__ E, float *__restrict__ Y, int accumulate)
 {
     for (int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x); i < MN; i += 4 * (int64_t)gridDim.x * 256) {
+        const int e = E[(uint32_t)i / N];   // in flight beside the partials
         f4 s = split_sum4(P + i, S, zs);
         if (N % 4 == 0) {
-            s = undo_row_exp4(s, E[(uint32_t)i / N]);
+            s = undo_row_exp4(s, e);
         } else {   // the four elements may lie in several rows (past the end: the last row's)
 #pragma unroll
             for (int j = 0; j < 4; ++j) s[j] = ldexpf(s[j], -E[(uint32_t)min<int64_t>(i + j, MN - 1) / N]);
@@ -833,7 +834,8 @@ split_k_rope_kernel(const float *__restrict__ P, int S, int64_t N, int64_t zs,
 #pragma clang fp contract(off)
     const int64_t m = blockIdx.y, n = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x), t = m * N + n;
     if (n >= N) return;
-    const f4 x = undo_row_exp4(split_sum4(P + t, S, zs), E[m]);
+    const int e = E[m];
+    const f4 x = undo_row_exp4(split_sum4(P + t, S, zs), e);
     const int64_t p = (int64_t)ra.start + (ra.pos ? *ra.pos : 0) + m;
     const bool in_table = p >= 0 && p < ra.table_rows, in_cache = in_table && p < ra.cache_rows;
     const int kind = n < ra.qd ? 0 : n < (int64_t)ra.qd + ra.kvd ? 1 : 2;
