@@ -1077,23 +1077,19 @@ int launch(aih_ctx *ctx, const uint8_t *W, int64_t N, int64_t K, int64_t row_byt
     const int64_t gx = (N + BN - 1) / BN, gy = (M + BM - 1) / BM, gy2 = (M + BM2 - 1) / BM2;
     const int64_t gy4 = (M + 2 * BM2 - 1) / (2 * BM2);
     if (gy > 65535 || gx > 0x7FFFFFFF) return AIH_E_LIMIT;
-    GemmPlan p = plan_gemm(ctx->cu_count, N, K, M, epi, may_split);
+    const GemmPlan p = plan_gemm(ctx->cu_count, N, K, M, epi, may_split);
     const int64_t zs = split_stride(M, N);
     void *ws = nullptr;
     if (p.splits > 1) {
+        // a shape that splits always splits: a workspace that cannot grow here
+        // (512-row tiles during a graph capture; 128-row tiles fit the one that
+        // aih_init sets aside) is an error, not a change of the order of the sum
         const size_t bytes = (size_t)p.splits * (size_t)zs * sizeof(float);
-        int rc = AIH_OK;
-        if (room && bytes <= room->bytes) ws = room->ptr;
-        else rc = room ? AIH_E_SCRATCH : aih_workspace2(ctx, bytes, &ws);
-        if (rc) {
-            // 512-row tiles: a shape that splits always splits (a workspace
-            // that cannot grow here, as during a graph capture, is an error).
-            // 128-row tiles: their partial sums fit the workspace that
-            // aih_init sets aside; without it the product runs whole.
-            if (p.tile != BM) return rc;
-            ws = nullptr;
-            p.splits = 1;
-            p.ssper = (int)((K / 64 + SC - 1) / SC);
+        if (room) {
+            if (bytes > room->bytes) return AIH_E_SCRATCH;
+            ws = room->ptr;
+        } else if (const int rc = aih_workspace2(ctx, bytes, &ws)) {
+            return rc;
         }
     }
     float *const P = static_cast<float *>(ws);

@@ -227,10 +227,15 @@ int aih_init(int device_index, aih_ctx **out)
         release(ctx);
         return (int)err;
     }
-    // room for the partial sums of GEMMs of at most 256 rows (plan_gemm), so
-    // that they split alike inside a graph capture; without it they run whole
+    // Room for the partial sums of GEMMs of at most 256 rows (plan_gemm), which
+    // split by their shape alone, inside a graph capture too: a context has it
+    // or does not come to be.
     void *reserved = nullptr;
-    (void)aih_workspace2(ctx, AIH_NOALLOC_SCRATCH_BYTES, &reserved);
+    const int ws = aih_workspace2(ctx, AIH_NOALLOC_SCRATCH_BYTES, &reserved);
+    if (ws != AIH_OK) {
+        release(ctx);
+        return ws;
+    }
     *out = ctx;
     return AIH_OK;
 }

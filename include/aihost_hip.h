@@ -109,8 +109,11 @@ typedef struct aih_device_info {
 
 /* ---- device / context (IComputeDevice, AIHost/AIHost/ICompute/IComputeDevice.cs:27-72) */
 
-/* Open device `device_index`, create its stream and the pinned staging ring.
- * Fails with AIH_E_NOT_GFX950 on any other architecture.
+/* Open device `device_index`, create its stream and the pinned staging ring,
+ * and set 17 MiB of device memory aside for the partial sums of GEMMs of at
+ * most 256 rows (aih_qgemm; held until aih_destroy, not in tracked_bytes).
+ * Fails with AIH_E_NOT_GFX950 on any other architecture, and with
+ * hipErrorOutOfMemory (2) where that memory cannot be had.
  * Replaces ROCmComputeDevice's constructor (AIHost/AIHost/ICompute/ROCm/ROCmComputeDevice.cs:15-50). */
 int aih_init(int device_index, aih_ctx **out);
 

@@ -5,6 +5,8 @@ Covers the prefill workload (Q4_K W 4096x4096, X 512x4096), every format,
 partial tiles in M and N, K of one step, the ComputeOps-style routing
 (M <= 8 -> matvec, larger -> GEMM) and argument errors.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -130,6 +132,46 @@ def test_small_grid_split_k(device, orc, qtype, n, k, m, offset):
             b.dispose()
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
     assert_close(got[0], orc.matvec(qtype, w, n, k, x, nthreads=16), TOL, "type %d %dx%d M=%d" % (qtype, n, k, m))
+
+
+def test_small_grid_split_k_captured_on_a_fresh_context(device):
+    # only the X workspace was grown before the capture (by a product that is
+    # not split): the partial sums have the room that aih_init sets aside; every
+    # replay, with eager work between, gives the eager bits of another context
+    L = nat.lib()
+    n, k, m = 1024, 4096, 64
+    if device.info().compute_units == 256:
+        assert nat.qgemm_plan(device.handle, n, k, m)[1] > 1
+        assert nat.qgemm_plan(device.handle, 16384, k, 300)[1] == 1
+    w = synth_weight(nat.Q4_K, n, k, seed=5)
+    x = x_of(m, k, seed=6)
+    ref = qgemm(device, nat.Q4_K, w, n, k, x)
+    fresh = C.HipComputeDevice(0)
+    graph = ctypes.c_void_p()
+    bufs = [upload(fresh, w), upload(fresh, x), fresh.create_buffer(m * n * 4), upload(fresh, synth_weight(nat.Q4_K, 16384, k)),
+            upload(fresh, x_of(300, k)), fresh.create_buffer(300 * 16384 * 4)]
+    wb, xb, yb, wl, xl, yl = (b.get_pointer() for b in bufs)
+    try:
+        h = fresh.handle
+        nat.check(L.aih_qgemm(h, nat.Q4_K, wl, 16384, k, xl, 300, yl), "large")
+        nat.check(L.aih_capture_begin(h), "capture")
+        st = L.aih_qgemm(h, nat.Q4_K, wb, n, k, xb, m, yb)
+        nat.check(L.aih_capture_end(h, ctypes.byref(graph)), "capture end")
+        nat.check(st, "captured")
+        for _ in range(3):
+            bufs[2].write(np.full(m * n, -7.0, np.float32))
+            nat.check(L.aih_graph_launch(h, graph.value), "replay")
+            fresh.synchronize()
+            got = bufs[2].read_range(0, m * n, np.float32).reshape(m, n)
+            assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+            nat.check(L.aih_qgemm(h, nat.Q4_K, wl, n, k, xl, 100, yl), "eager, split too")
+            fresh.synchronize()
+    finally:
+        if graph.value:
+            L.aih_graph_destroy(graph.value)
+        for b in bufs:
+            b.dispose()
+        fresh.dispose()
 
 
 # The 512 x 128 tiles of large products: row and column remainders, a second
