@@ -73,6 +73,7 @@ SIGNATURES = {
     "aih_qgemm_qkv_rope": (_i, [_vp, _i, _vp, _i64, _vp, _vp, _f, _i64, _i, _vp, _vp, _vp, ctypes.c_int32,
                                 ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _vp, _vp, ctypes.c_int32, _i64]),
     "aih_operand_bytes": (_i64, [_i64, _i64]),
+    "aih_qgemm_tile_columns": (_i, [_vp, _i64, _i64, _i64, _i]),
     "aih_qgemm_plan": (_i, [_vp, _i64, _i64, _i64, _i, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]),
     "aih_matmul_weights_q_noalloc": (_i, [_vp, _i, _vp, _i64, _i64, _vp, _i64, _vp]),
     "aih_probe_stream_read": (_i, [_vp, _vp, _u64, _i, _vp]),
@@ -91,6 +92,7 @@ SIGNATURES = {
     "aih_attention_scratch_floats": (_i64, [ctypes.c_int32, ctypes.c_int32]),
     "aih_attention": (_i, [_vp, _vp, _vp, _vp, _vp, _i64, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
                            ctypes.c_int32, _vp, ctypes.c_int32, _f, _vp, _i64]),
+    "aih_attention_heads_per_workgroup": (_i, [_vp, _i64, _i, _i, _i, _i]),
     "aih_attention_strided": (_i, [_vp, _vp, _i64, _vp, _vp, _vp, _i64, ctypes.c_int32, ctypes.c_int32,
                                    ctypes.c_int32, ctypes.c_int32, _vp, ctypes.c_int32, _f, _vp, _i64]),
     "aih_attention_operand": (_i, [_vp, _vp, _i64, _vp, _vp, _vp, _i64, ctypes.c_int32, ctypes.c_int32,
@@ -159,6 +161,12 @@ def qgemm_plan(handle, n, k, m, may_split=True):
     check(lib().aih_qgemm_plan(handle, int(n), int(k), int(m), int(bool(may_split)), ctypes.byref(t),
                                ctypes.byref(s)), "aih_qgemm_plan")
     return t.value, s.value
+
+
+def qgemm_tile(handle, n, k, m, may_split=True):
+    """(tile rows, tile columns, K splits) of the same plan."""
+    rows, splits = qgemm_plan(handle, n, k, m, may_split)
+    return rows, lib().aih_qgemm_tile_columns(handle, int(n), int(k), int(m), int(bool(may_split))), splits
 
 
 def check(status, what):

@@ -2324,7 +2324,8 @@ int aih_add(aih_ctx *ctx, const float *A, const float *B, float *Y, int64_t n)
 // schedule of the query tiles' workgroups over the CUs, in key tiles (the
 // longest workgroup, the mean load, and k + 1 workgroups at least as long as
 // the (k cus + 1)-th on some CU), at the measured 3.45 us a tile for two heads
-// and 2.45 us for one.  A position in device memory counts as 0.  Measured at
+// and 2.45 us for one.  A position in device memory counts as 0: the host cannot
+// know it, and one head at a time is never slower than it was.  Measured at
 // 32 heads, one -> two: 512 queries 28.9 -> 40.3 us (128 workgroups on 256
 // CUs), 1024 59 -> 69, 1500 119 -> 94.  Over 91 shapes (4 to 64 heads, 9 to
 // 2048 queries, positions 0 to 3000) it picks the faster one, or a tie.
@@ -2345,6 +2346,14 @@ static bool prefill_pairs(const aih_ctx *ctx, int64_t n_q, int32_t n_heads, int3
         return most;
     };
     return 3.45 * load(n_heads / 2) < 2.45 * load(n_heads);
+}
+
+int aih_attention_heads_per_workgroup(aih_ctx *ctx, int64_t n_q, int32_t n_heads, int32_t n_kv_heads, int32_t start,
+                                      int32_t max_len)
+{
+    if (!ctx || n_q < 2 || n_heads <= 0 || n_kv_heads <= 0 || n_heads % n_kv_heads || start < 0 || max_len <= 0)
+        return AIH_E_INVALID;
+    return prefill_pairs(ctx, n_q, n_heads, n_kv_heads, start, max_len) ? 2 : 1;
 }
 
 // The tiled (prefill) attention: the output as fp32 rows in O, or, with Xt,

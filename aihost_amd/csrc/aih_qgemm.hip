@@ -1175,3 +1175,9 @@ extern "C" int aih_qgemm_plan(aih_ctx *ctx, int64_t N, int64_t K, int64_t M, int
     *splits = p.splits;
     return AIH_OK;
 }
+
+extern "C" int aih_qgemm_tile_columns(aih_ctx *ctx, int64_t N, int64_t K, int64_t M, int may_split)
+{
+    if (!ctx || N <= 0 || M <= 0 || K <= 0 || K % BK) return AIH_E_INVALID;
+    return plan_gemm(ctx->cu_count, N, K, M, kEpiStore, may_split != 0).cols;
+}

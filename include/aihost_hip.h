@@ -266,13 +266,18 @@ int aih_qgemm(aih_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
 
 /* The tiling aih_qgemm and aih_qgemm_fused choose for an M x K by N product
  * on this context's device: rows per workgroup tile (128, 256 or 512) and
- * the number of K splits (1 = none), for a call that may split
- * (may_split != 0: aih_qgemm, aih_qgemm_fused with AIH_POST_STORE or
- * AIH_POST_ACCUMULATE) or may not (aih_matmul_weights_q and its
- * allocation-free twin).  K a multiple of 64.  No counterpart in the
+ * the number of K splits (1 = none).  Products of more than 256 rows split only
+ * in calls that may (may_split != 0: aih_qgemm, aih_qgemm_fused with
+ * AIH_POST_STORE or AIH_POST_ACCUMULATE; not aih_matmul_weights_q, its
+ * allocation-free twin and the other epilogues); smaller ones split alike in
+ * every call, whatever may_split.  K a multiple of 64.  No counterpart in the
  * reference: it lets tests and tools see which kernel a shape reaches. */
 int aih_qgemm_plan(aih_ctx *ctx, int64_t N, int64_t K, int64_t M, int may_split, int32_t *tile_rows,
                    int32_t *splits);
+
+/* The columns per workgroup tile of the same plan (64, or 128 beside 512
+ * rows), or a negative status. */
+int aih_qgemm_tile_columns(aih_ctx *ctx, int64_t N, int64_t K, int64_t M, int may_split);
 
 /* ComputeOps.MatMulWeights semantics for a quantized weight: routes M <= 8 to
  * aih_qmatvec and larger M to aih_qgemm; more than 256 rows are never split
@@ -443,6 +448,16 @@ int64_t aih_attention_scratch_floats(int32_t n_heads, int32_t max_len);
 int aih_attention(aih_ctx *ctx, const float *Q, const float *Kc, const float *Vc, float *O, int64_t n_q,
                   int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, int32_t start, const int32_t *pos,
                   int32_t max_len, float scale, float *scratch, int64_t scratch_floats);
+
+/* The query heads of one KV head that a workgroup of aih_attention (and its
+ * variants below) takes for n_q > 1 rows from position `start` over a cache of
+ * max_len rows: 1 or 2, by whichever schedule of workgroups over the device's
+ * CUs is shorter; or a negative status.  The two add a row's keys up in another
+ * order.  A position in device memory is not known when the kernel is chosen
+ * and counts as 0, so a row's last bits can differ between a call with `start`
+ * and one with the same position in *pos.  No counterpart in the reference. */
+int aih_attention_heads_per_workgroup(aih_ctx *ctx, int64_t n_q, int32_t n_heads, int32_t n_kv_heads, int32_t start,
+                                      int32_t max_len);
 
 /* aih_attention with query rows ldq floats apart (ldq >= n_heads*head_dim,
  * a multiple of 4): the query block of a fused Q|K|V projection output read

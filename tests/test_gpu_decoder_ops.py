@@ -271,7 +271,13 @@ def test_attention_decode_scratch_reused(device, bufs):
 def test_attention_prefill(device, bufs, n_q, start):
     # query tiles of 64 and key tiles of 64: full and partial tiles of both,
     # rows that end at the cache's last row (start + n_q = 640)
+    _assert_heads(device, 1, n_q, 32, 8, start, 640)
     _attn(device, bufs, n_q, start, 640)
+
+
+def _assert_heads(device, heads, n_q, nh, nkv, start, max_len):
+    if device.info().compute_units == 256:
+        assert L.aih_attention_heads_per_workgroup(device.handle, n_q, nh, nkv, start, max_len) == heads
 
 
 # enough query tiles and heads for two heads per workgroup (on a 256-CU
@@ -279,6 +285,7 @@ def test_attention_prefill(device, bufs, n_q, start):
 # position; the first rows of each see no key of the second half of a tile
 @pytest.mark.parametrize("n_q,start,nh,nkv,pos", [(800, 0, 64, 8, None), (709, 77, 64, 32, None), (770, 0, 96, 6, 50)])
 def test_attention_prefill_head_pairs(device, bufs, n_q, start, nh, nkv, pos):
+    _assert_heads(device, 2, n_q, nh, nkv, start, start + (pos or 0) + n_q)
     _attn(device, bufs, n_q, start, start + (pos or 0) + n_q, nh, nkv, pos)
 
 
@@ -286,6 +293,7 @@ def test_attention_prefill_head_pairs_magnitudes(device, bufs):
     # as below, with V tiles from 1e-6 to 1e6 row by row, and bit for bit
     # under powers of two
     nh, nkv, n_q = 64, 8, 800
+    _assert_heads(device, 2, n_q, nh, nkv, 0, n_q)
     q, K, V = rnd(71, n_q, nh * 128), rnd(72, n_q, nkv * 128), rnd(73, n_q, nkv * 128)
     V *= (10.0 ** (3 * ((np.arange(n_q) // 64) % 5 - 2))).astype(np.float32)[:, None]
     q *= (10.0 ** -(np.arange(n_q) % 4)).astype(np.float32)[:, None]
@@ -304,6 +312,7 @@ def test_attention_prefill_head_pairs_large_values_of_small_weight(device, bufs,
     # they must not take bits from the keys that make up the result (rows from
     # 64 on, 1e-5 as above)
     nh, nkv, n_q = 64, 8, 800
+    _assert_heads(device, 2, n_q, nh, nkv, 0, n_q)
     q, K, V = rnd(81, n_q, nh * 128), rnd(82, n_q, nkv * 128), rnd(83, n_q, nkv * 128)
     q[:, ::128] = 8.0
     K[:, ::128] = 0.0
@@ -388,6 +397,8 @@ def test_attention_argument_errors(device, bufs):
     assert L.aih_attention(h, X, X, X, X, 1, 32, 8, 64, 0, None, 8, 1.0, X, 4096) == nat.AIH_E_UNSUPPORTED
     assert L.aih_attention(h, X, X, X, X, 1, 32, 5, 128, 0, None, 8, 1.0, X, 4096) == nat.AIH_E_INVALID
     assert L.aih_attention(h, X, X, X, X, 4, 32, 8, 128, 6, None, 8, 1.0, X, 4096) == nat.AIH_E_LIMIT
+    assert L.aih_attention_heads_per_workgroup(h, 4, 32, 5, 0, 8) == nat.AIH_E_INVALID
+    assert L.aih_attention_heads_per_workgroup(h, 1, 32, 8, 0, 8) == nat.AIH_E_INVALID
     assert L.aih_attention(h, X, X, X, X, 1, 32, 8, 128, 0, None, 8, 1.0, None, 0) == nat.AIH_E_INVALID
     device.synchronize()
 

@@ -50,20 +50,24 @@ def test_shapes(device, orc, qtype, n, k, m):
 
 
 # Grids large enough for the 256-row tiles on a 256-CU device (fewer rounds of
-# workgroups than the 128-row tiles), and the 512-row tiles of the largest
-# grids: partial tiles in M and N, and for Q8_0 a partial last super-step.
-@pytest.mark.parametrize("qtype,n,k,m", [
-    (nat.Q4_K, 6377, 1536, 300), (nat.Q6_K, 6400, 1024, 384),
-    (nat.Q8_0, 6377, 1600, 300), (nat.Q4_0, 6400, 1600, 257),
-    # 512-row tiles (more than 256 rows over 447-448 column tiles)
-    (nat.Q4_K, 28600, 512, 300), (nat.Q6_K, 28672, 768, 512),
-    (nat.Q8_0, 28000, 832, 450), (nat.Q4_0, 28672, 576, 257),
+# workgroups than the 128-row tiles), and the 512 x 64 and 512 x 128 tiles of the
+# largest grids: partial tiles in M and N, and for Q8_0 and Q4_0 a partial last
+# super-step.
+@pytest.mark.parametrize("qtype,n,k,m,tile", [
+    (nat.Q4_K, 6377, 1536, 300, (256, 64, 1)), (nat.Q6_K, 6400, 1024, 384, (256, 64, 1)),
+    (nat.Q8_0, 6377, 1600, 300, (256, 64, 1)), (nat.Q4_0, 6400, 1600, 257, (256, 64, 1)),
+    # more than 256 rows over 219-224 tiles of 64 columns
+    (nat.Q4_K, 14300, 1536, 300, (512, 64, 1)), (nat.Q6_K, 14336, 1024, 512, (512, 64, 1)),
+    (nat.Q8_0, 14000, 832, 450, (512, 64, 1)), (nat.Q4_0, 14301, 1600, 333, (512, 64, 1)),
+    # and over 447-448
+    (nat.Q4_K, 28600, 512, 300, (512, 128, 1)), (nat.Q6_K, 28672, 768, 512, (512, 128, 1)),
+    (nat.Q8_0, 28000, 832, 450, (512, 128, 1)), (nat.Q4_0, 28672, 576, 257, (512, 128, 1)),
 ])
-def test_wide_tiles(device, orc, qtype, n, k, m):
-    tile, splits = nat.qgemm_plan(device.handle, n, k, m)
-    want = 512 if n > 20000 else 256
-    if (tile, splits) != (want, 1):
-        pytest.skip("on this device's CU count the shape takes %d-row tiles, %d splits" % (tile, splits))
+def test_wide_tiles(device, orc, qtype, n, k, m, tile):
+    if device.info().compute_units == 256:
+        assert nat.qgemm_tile(device.handle, n, k, m) == tile
+    elif nat.qgemm_tile(device.handle, n, k, m) != tile:
+        pytest.skip("another tiling on this device's CU count")
     w = synth_weight(qtype, n, k, seed=n + k)
     x = x_of(m, k, seed=m * 3 + k)
     y = qgemm(device, qtype, w, n, k, x)
@@ -175,23 +179,26 @@ def test_small_grid_split_k_captured_on_a_fresh_context(device):
 
 
 # The 512 x 128 tiles of large products: row and column remainders, a second
-# column half past N, 64-k remainders, one super-step.  A row's bits do not
-# depend on the tiling, so the product equals the one taken 300 rows at a time
-# (128-row tiles on a 256-CU device).
-@pytest.mark.parametrize("qtype,n,k,m", [(nat.Q4_K, 8150, 512, 1537), (nat.Q6_K, 14300, 768, 1000),
-                                         (nat.Q8_0, 28600, 192, 500), (nat.Q4_0, 8129, 1344, 2048)])
+# column half past N, 64-k remainders, one super-step and up to 9.  A row's bits
+# do not depend on the tiling, so the product equals the one taken 128 rows at a
+# time, in unsplit 128-row tiles (held to the oracle above).
+@pytest.mark.parametrize("qtype,n,k,m", [(nat.Q4_K, 8150, 512, 1580), (nat.Q6_K, 14300, 768, 1000),
+                                         (nat.Q8_0, 28600, 192, 500), (nat.Q4_0, 8129, 1344, 2048),
+                                         (nat.Q4_K, 14300, 2304, 1000)])
 def test_wide_tiles_equal_row_chunks(device, qtype, n, k, m):
     if device.info().compute_units == 256:
-        assert nat.qgemm_plan(device.handle, n, k, m, may_split=False) == (512, 1)
+        assert nat.qgemm_tile(device.handle, n, k, m, may_split=False) == (512, 128, 1)
+        for rows in {128, m % 128} - {0}:
+            assert rows > 8 and nat.qgemm_tile(device.handle, n, k, rows, may_split=False) == (128, 64, 1)
     wb, xb = upload(device, synth_weight(qtype, n, k, seed=n + k)), upload(device, x_of(m, k, seed=m))
     yb, cb = device.create_buffer(m * n * 4 + 32), device.create_buffer(m * n * 4)
     f = nat.lib().aih_matmul_weights_q
     try:
         yb.write(np.full(m * n + 8, -7.0, np.float32))
         nat.check(f(device.handle, int(qtype), wb.get_pointer(), n, k, xb.get_pointer(), m, yb.get_pointer()), "wide")
-        for r in range(0, m, 300):
+        for r in range(0, m, 128):
             nat.check(f(device.handle, int(qtype), wb.get_pointer(), n, k, xb.get_pointer() + r * k * 4,
-                        min(300, m - r), cb.get_pointer() + r * n * 4), "rows")
+                        min(128, m - r), cb.get_pointer() + r * n * 4), "rows")
         y, c = yb.read_range(0, m * n + 8, np.float32), cb.read_range(0, m * n, np.float32)
     finally:
         for b in (wb, xb, yb, cb):

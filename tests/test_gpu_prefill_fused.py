@@ -264,11 +264,19 @@ def test_qkv_rope_gemm_with_split_k(device, m, start, dpos, trows, crows):
                                              norm=1e6)
 
 
-# both fused epilogues over the 512 x 128 tiles (N = 6144 and 8064)
+# both fused epilogues over the 512 x 64 tiles (N = 14336)
+def test_epilogues_of_the_512x64_tiles(device):
+    if device.info().compute_units == 256:
+        assert nat.qgemm_tile(device.handle, 14336, 256, 400, may_split=False) == (512, 64, 1)
+    test_qkv_rope_gemm_equals_gemm_then_rope(device, 96, 8, 256, 400, 3, None, 512, 403, nat.PRE_RMSNORM, nat.Q4_K)
+    test_silu_pairs_operand_chain_equals_separate_operators(device, 256, 7168, 400, nat.Q8_0)
+
+
+# and over the 512 x 128 tiles (N = 6144 and 8064)
 def test_epilogues_of_the_wide_tiles(device):
     if device.info().compute_units == 256:
-        assert nat.qgemm_plan(device.handle, 6144, 256, 2000) == (512, 1)
-        assert nat.qgemm_plan(device.handle, 8064, 256, 1537) == (512, 1)
+        assert nat.qgemm_tile(device.handle, 6144, 256, 2000, may_split=False) == (512, 128, 1)
+        assert nat.qgemm_tile(device.handle, 8064, 256, 1537, may_split=False) == (512, 128, 1)
     test_qkv_rope_gemm_equals_gemm_then_rope(device, 32, 8, 256, 2000, 3, None, 2048, 2040, nat.PRE_RMSNORM, nat.Q4_K)
     test_silu_pairs_operand_chain_equals_separate_operators(device, 256, 4032, 1537, nat.Q8_0)
 
@@ -354,6 +362,8 @@ def test_attention_operand_of_head_pairs(device):
     device): the operand is the fp32 output rounded, its exponents zero."""
     L, h = nat.lib(), device.handle
     n_q, nh, nkv, qd = 801, 64, 8, 64 * 128
+    if device.info().compute_units == 256:
+        assert L.aih_attention_heads_per_workgroup(h, n_q, nh, nkv, 0, n_q) == 2
     rng = np.random.default_rng(17)
     bufs = [upload(device, rng.standard_normal((n_q, w * 128)).astype(np.float32)) for w in (nh, nkv, nkv)]
     q, kb, vb = (b.get_pointer() for b in bufs)
