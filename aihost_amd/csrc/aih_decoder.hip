@@ -1222,12 +1222,16 @@ __device__ __forceinline__ float xor_lanes_max(float v)   // over lanes l, l^16,
     return fmaxf(v, __shfl_xor(v, 32));
 }
 
-// One tile of one KV head in registers, as the 256 threads of a workgroup
-// load it: K thread (keys kt_key + 16i, dims 8 kt_ch .. +7), V thread (dims
-// 4 vt_dq .. +3 of the 8 keys of slots 32 vt_t + 8 vt_g .. +7); rows past
+// One tile of one KV head in registers, as TH (256 or 512) threads load it: K
+// thread (keys kt_key + TH/16 i, dims 8 kt_ch .. +7), V thread (dims
+// VD vt_d .. + VD - 1 of the 8 keys of slots 32 vt_t + 8 vt_g .. +7); rows past
 // p_last are zeros.
+template <int TH>
 struct KVTile {
-    f4 kr[8], vr[8];
+    static constexpr int KN = 1024 / TH, VD = 1024 / TH, NW = TH / 64;   // keys, V dims per thread; waves
+    typedef float VV __attribute__((ext_vector_type(VD)));
+    f4 kr[2 * KN];
+    VV vr[8];
 
     __device__ __forceinline__ void load(const float *__restrict__ Kc, const float *__restrict__ Vc,
                                          int64_t kv_stride, int kvh, int64_t j0, int64_t p_last, int tid)
@@ -1241,29 +1245,33 @@ struct KVTile {
         const int64_t base = j0 * kv_stride + kvh * kHD;
         const Rsrc rk = make_rsrc(uniform_ptr(Kc + base), bytes), rv = make_rsrc(uniform_ptr(Vc + base), bytes);
         const int kt_key = tid >> 4, kt_ch = tid & 15;
-        const int vt_t = tid >> 7, vt_g = (tid >> 5) & 3, vt_dq = tid & 31;
+        const int vt_t = tid / (TH / 2), vt_g = tid / (TH / 8) & 3, vt_d = tid % (TH / 8);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t at = (uint32_t)(kt_key + 16 * i) * row + 32 * kt_ch;
+        for (int i = 0; i < KN; ++i) {
+            const uint32_t at = (uint32_t)(kt_key + TH / 16 * i) * row + 32 * kt_ch;
             kr[2 * i] = bld16(rk, at);
             kr[2 * i + 1] = bld16(rk, at + 16);
         }
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-            vr[e] = bld16(rv, (uint32_t)(32 * vt_t + 16 * (e / 4) + 4 * vt_g + e % 4) * row + 16 * vt_dq);
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t at = (uint32_t)(32 * vt_t + 16 * (e / 4) + 4 * vt_g + e % 4) * row + 4 * VD * vt_d;
+            if constexpr (VD == 4) vr[e] = bld16(rv, at);
+            else vr[e] = bld8(rv, at);
+        }
     }
 
     // this wave's max |K| and |V|, into tmax[0][w] and tmax[1][w]
-    __device__ __forceinline__ void wave_max(float (*tmax)[4], int lane, int w) const
+    __device__ __forceinline__ void wave_max(float (*tmax)[NW], int lane, int w) const
     {
         float mk = 0.f, mv = 0.f;
 #pragma unroll
+        for (int i = 0; i < 2 * KN; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) mk = fmaxf(mk, fabsf(kr[i][u]));
+#pragma unroll
         for (int i = 0; i < 8; ++i)
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                mk = fmaxf(mk, fabsf(kr[i][u]));
-                mv = fmaxf(mv, fabsf(vr[i][u]));
-            }
+            for (int u = 0; u < VD; ++u) mv = fmaxf(mv, fabsf(vr[i][u]));
         mk = xor_lanes_max(row16_max(mk));
         mv = xor_lanes_max(row16_max(mv));
         if (lane == 0) {
@@ -1272,37 +1280,40 @@ struct KVTile {
         }
     }
 
-    // this thread's 16 split chunks into the padded LDS images (K hi, K lo,
+    // the exponent of the tile's maximum, from all waves' (which: 0 K, 1 V)
+    __device__ static __forceinline__ int split_exp_of(const float (*tmax)[NW], int which)
+    {
+        float m = tmax[which][0];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) m = fmaxf(m, tmax[which][w]);
+        return split_exp(m);
+    }
+
+    // this thread's split chunks into the padded LDS images (K hi, K lo,
     // V^T hi, V^T lo from lds)
     __device__ __forceinline__ void split_to_lds(int ek, int ev, int tid, _Float16 *lds) const
     {
         const int kt_key = tid >> 4, kt_ch = tid & 15;
-        const int vt_t = tid >> 7, vt_g = (tid >> 5) & 3, vt_dq = tid & 31;
+        const int vt_t = tid / (TH / 2), vt_g = tid / (TH / 8) & 3, vt_d = tid % (TH / 8);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < KN; ++i) {
             h8 hi, lo;
             split8(kr[2 * i], kr[2 * i + 1], ek, hi, lo);
-            _Float16 *at = lds + (kt_key + 16 * i) * kRKH + 8 * kt_ch;
+            _Float16 *at = lds + (kt_key + TH / 16 * i) * kRKH + 8 * kt_ch;
             *reinterpret_cast<h8 *>(at) = hi;
             *reinterpret_cast<h8 *>(at + kKT * kRKH) = lo;
         }
 #pragma unroll
-        for (int d = 0; d < 4; ++d) {
+        for (int d = 0; d < VD; ++d) {
             h8 hi, lo;
             split8(f4{vr[0][d], vr[1][d], vr[2][d], vr[3][d]}, f4{vr[4][d], vr[5][d], vr[6][d], vr[7][d]}, ev, hi,
                    lo);
-            _Float16 *at = lds + 2 * kKT * kRKH + (4 * vt_dq + d) * kRVH + 32 * vt_t + 8 * vt_g;
+            _Float16 *at = lds + 2 * kKT * kRKH + (VD * vt_d + d) * kRVH + 32 * vt_t + 8 * vt_g;
             *reinterpret_cast<h8 *>(at) = hi;
             *reinterpret_cast<h8 *>(at + kHD * kRVH) = lo;
         }
     }
 };
-
-__device__ __forceinline__ int split_exp_of(const float (*tmax)[4], int which)
-{
-    return split_exp(fmaxf(fmaxf(tmax[which][0], tmax[which][1]), fmaxf(tmax[which][2], tmax[which][3])));
-}
-
 
 // Four consecutive values k0 .. k0 + 3 (k0 % 4 == 0) of row m of a GEMM
 // operand with K columns, rounded to fp16 into its MFMA fragment-order image
@@ -1418,7 +1429,8 @@ attn_prefill_kernel(const float *__restrict__ Q, int64_t ldq, const float *__res
     // the next tile's rows in registers; both halves take n_iter steps (a
     // half whose range has ended idles through its last ones), so that the
     // workgroup barriers line up
-    KVTile kv;
+    typedef KVTile<256> Tile;
+    Tile kv;
     if (j_begin < j_end) {
         kv.load(Kc, Vc, kv_stride, kvh, j_begin, p_last, ht);
         kv.wave_max(tmax, lane, w);
@@ -1427,7 +1439,7 @@ attn_prefill_kernel(const float *__restrict__ Q, int64_t ldq, const float *__res
         const int64_t j0 = j_begin + kKT * it;
         const bool act = j0 < j_end;
         __syncthreads();   // the previous tile is consumed; tmax holds this one's maxima
-        const int ek = split_exp_of(tmax, 0), ev = split_exp_of(tmax, 1);
+        const int ek = Tile::split_exp_of(tmax, 0), ev = Tile::split_exp_of(tmax, 1);
         if (act) kv.split_to_lds(ek, ev, ht, lds);
         __syncthreads();
         if (!act) continue;
@@ -1540,111 +1552,27 @@ attn_prefill_kernel(const float *__restrict__ Q, int64_t ldq, const float *__res
     prefill_operand_rows(Xt, r, i, n_q, q_stride, h, g);
 }
 
-// One tile of one KV head in registers, as the 512 threads of a workgroup
-// load it: K thread (keys kt_key + 32i, dims 8 kt_ch .. +7), V thread (dims
-// 2 vt_dp, + 1 of the 8 keys of slots 32 vt_t + 8 vt_g .. +7); rows past
-// p_last are zeros.
-struct KVTile512 {
-    f4 kr[4];
-    fl2 vr[8];
-
-    __device__ __forceinline__ void load(const float *__restrict__ Kc, const float *__restrict__ Vc,
-                                         int64_t kv_stride, int kvh, int64_t j0, int64_t p_last, int tid)
-    {
-        // one buffer per tile over its rows up to p_last: the rows past it
-        // (all of them when p_last < j0, as for a position before the
-        // cache) load as zeros
-        const uint32_t row = (uint32_t)kv_stride * 4;
-        const int64_t valid = max<int64_t>(0, min<int64_t>(p_last + 1 - j0, kKT));
-        const uint32_t bytes = __builtin_amdgcn_readfirstlane((uint32_t)valid * row);
-        const int64_t base = j0 * kv_stride + kvh * kHD;
-        const Rsrc rk = make_rsrc(uniform_ptr(Kc + base), bytes), rv = make_rsrc(uniform_ptr(Vc + base), bytes);
-        const int kt_key = tid >> 4, kt_ch = tid & 15;
-        const int vt_t = tid >> 8, vt_g = (tid >> 6) & 3, vt_dp = tid & 63;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const uint32_t at = (uint32_t)(kt_key + 32 * i) * row + 32 * kt_ch;
-            kr[2 * i] = bld16(rk, at);
-            kr[2 * i + 1] = bld16(rk, at + 16);
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            vr[e] = bld8(rv, (uint32_t)(32 * vt_t + 16 * (e / 4) + 4 * vt_g + e % 4) * row + 8 * vt_dp);
-    }
-
-    // this wave's max |K| and |V|, into tmax[0][w] and tmax[1][w]
-    __device__ __forceinline__ void wave_max(float (*tmax)[8], int lane, int w) const
-    {
-        float mk = 0.f, mv = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int u = 0; u < 4; ++u) mk = fmaxf(mk, fabsf(kr[i][u]));
-#pragma unroll
-        for (int i = 0; i < 8; ++i) mv = fmaxf(mv, fmaxf(fabsf(vr[i].x), fabsf(vr[i].y)));
-        mk = xor_lanes_max(row16_max(mk));
-        mv = xor_lanes_max(row16_max(mv));
-        if (lane == 0) {
-            tmax[0][w] = mk;
-            tmax[1][w] = mv;
-        }
-    }
-
-    // this thread's split chunks into the padded LDS images (K hi, K lo,
-    // V^T hi, V^T lo from lds)
-    __device__ __forceinline__ void split_to_lds(int ek, int ev, int tid, _Float16 *lds) const
-    {
-        const int kt_key = tid >> 4, kt_ch = tid & 15;
-        const int vt_t = tid >> 8, vt_g = (tid >> 6) & 3, vt_dp = tid & 63;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            h8 hi, lo;
-            split8(kr[2 * i], kr[2 * i + 1], ek, hi, lo);
-            _Float16 *at = lds + (kt_key + 32 * i) * kRKH + 8 * kt_ch;
-            *reinterpret_cast<h8 *>(at) = hi;
-            *reinterpret_cast<h8 *>(at + kKT * kRKH) = lo;
-        }
-#pragma unroll
-        for (int d = 0; d < 2; ++d) {
-            h8 hi, lo;
-            split8(f4{vr[0][d], vr[1][d], vr[2][d], vr[3][d]}, f4{vr[4][d], vr[5][d], vr[6][d], vr[7][d]}, ev, hi,
-                   lo);
-            _Float16 *at = lds + 2 * kKT * kRKH + (2 * vt_dp + d) * kRVH + 32 * vt_t + 8 * vt_g;
-            *reinterpret_cast<h8 *>(at) = hi;
-            *reinterpret_cast<h8 *>(at + kHD * kRVH) = lo;
-        }
-    }
-};
-
-__device__ __forceinline__ int split_exp_of(const float (*tmax)[8], int which)
-{
-    float m = tmax[which][0];
-#pragma unroll
-    for (int w = 1; w < 8; ++w) m = fmaxf(m, tmax[which][w]);
-    return split_exp(m);
-}
-
-// The same products for NB heads of one KV head at once, where that still
+// The same products for two heads of one KV head at once, where that still
 // fills the CUs (prefill_pairs).  attn_prefill_kernel is bound by the splitting
 // of K and V into fp16 pairs (352 of 586 VALU instructions per wave and tile)
 // and by its LDS reads (64 KB per wave and tile for 96 MFMAs).  Here a
 // workgroup's eight waves share one image of a 64-key tile (each thread splits
 // half as much, and holds half as many rows in flight), and every K and V
-// fragment feeds the queries of NB heads.  Wave w of half h owns the queries
+// fragment feeds the queries of both heads.  Wave w of half h owns the queries
 // 16w .. 16w + 15 of each head and the keys 32h .. 32h + 31 of every tile (score
 // blocks 2h, 2h + 1, product step t = h); the halves merge at the end as above.
 // Two images in LDS, one barrier per tile.
-// On MI355X, NB = 2, 32 heads over 8: 2048 queries 188 -> 142 us, 1024 at
+// On MI355X, 32 heads over 8: 2048 queries 188 -> 142 us, 1024 at
 // position 2000 215 -> 179, 2048 at 2000 492 -> 363; 3.45 us a tile and
-// workgroup against 2.45 for one head.  With NB = 1 it is 3-5% slower than
-// attn_prefill_kernel, which therefore stays for one head at a time.
-template <int NB>
+// workgroup against 2.45 for one head.  The same form with one head (NB = 1) is
+// 3-5% slower than attn_prefill_kernel, which therefore stays for it.
 __global__ void __launch_bounds__(512, 1)
-attn_prefill_group_kernel(const float *__restrict__ Q, int64_t ldq, const float *__restrict__ Kc,
+attn_prefill_pair_kernel(const float *__restrict__ Q, int64_t ldq, const float *__restrict__ Kc,
                           const float *__restrict__ Vc, float *__restrict__ O, int64_t n_q, int32_t n_heads,
                           int32_t n_kv_heads, int32_t start, const int32_t *pos, int32_t max_len, float scale,
                           _Float16 *__restrict__ Xt)
 {
+    constexpr int NB = 2;   // heads
     // two tile images of K hi, K lo, V^T hi, V^T lo
     constexpr int kImage = 2 * kKT * kRKH + 2 * kHD * kRVH;
     __shared__ __align__(16) _Float16 lds2[2][kImage];
@@ -1712,14 +1640,15 @@ attn_prefill_group_kernel(const float *__restrict__ Q, int64_t ldq, const float 
     // tile t: its rows are loaded during tile t - 2, split into image t % 2
     // with the exponents of its maxima at the start of tile t - 1 (one
     // barrier per tile)
-    KVTile512 kv;
+    typedef KVTile<512> Tile;
+    Tile kv;
     int ek = 0, ev = 0;
     if (n_kt > 0) {
         kv.load(Kc, Vc, kv_stride, kvh, 0, p_last, tid);
         kv.wave_max(tmax[0], lane, wave);
         __syncthreads();
-        ek = split_exp_of(tmax[0], 0);
-        ev = split_exp_of(tmax[0], 1);
+        ek = Tile::split_exp_of(tmax[0], 0);
+        ev = Tile::split_exp_of(tmax[0], 1);
         kv.split_to_lds(ek, ev, tid, lds2[0]);
         if (n_kt > 1) {
             kv.load(Kc, Vc, kv_stride, kvh, kKT, p_last, tid);
@@ -1732,8 +1661,8 @@ attn_prefill_group_kernel(const float *__restrict__ Q, int64_t ldq, const float 
         const _Float16 *const ksh = lds2[it & 1], *const vsh = ksh + 2 * kKT * kRKH;
         int ek_next = 0, ev_next = 0;
         if (it + 1 < n_kt) {
-            ek_next = split_exp_of(tmax[(it + 1) & 1], 0);
-            ev_next = split_exp_of(tmax[(it + 1) & 1], 1);
+            ek_next = Tile::split_exp_of(tmax[(it + 1) & 1], 0);
+            ev_next = Tile::split_exp_of(tmax[(it + 1) & 1], 1);
             kv.split_to_lds(ek_next, ev_next, tid, lds2[(it + 1) & 1]);
             if (it + 2 < n_kt) kv.load(Kc, Vc, kv_stride, kvh, j0 + 2 * kKT, p_last, tid);   // in flight
         }
@@ -2365,7 +2294,7 @@ static int prefill_attention(aih_ctx *ctx, const float *Q, int64_t ldq, const fl
     const int64_t tiles = (n_q + kQTile - 1) / kQTile;
     if (tiles > 65535) return AIH_E_LIMIT;
     if (prefill_pairs(ctx, n_q, n_heads, n_kv_heads, start, max_len))
-        hipLaunchKernelGGL(attn_prefill_group_kernel<2>, dim3(n_heads / 2, (unsigned)tiles), dim3(512), 0, ctx->stream, Q,
+        hipLaunchKernelGGL(attn_prefill_pair_kernel, dim3(n_heads / 2, (unsigned)tiles), dim3(512), 0, ctx->stream, Q,
                            ldq, Kc, Vc, O, n_q, n_heads, n_kv_heads, start, pos, max_len, scale, Xt);
     else
         hipLaunchKernelGGL(attn_prefill_kernel, dim3(n_heads, (unsigned)tiles), dim3(512), 0, ctx->stream, Q, ldq,
