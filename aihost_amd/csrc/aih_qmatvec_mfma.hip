@@ -291,8 +291,8 @@ __device__ __forceinline__ float pair_scale(const PairRaw<NW> &r, int q, int g, 
 struct UQ80 {
     static constexpr int kBytes = 272, kBlocks = 8, kBlockElems = 32, SB = 32;
     static constexpr bool kOwner = true;
-    static constexpr bool kOwnMin = false;      // o = 128 d = 512 k
-    static constexpr float kSumScale = -512.f, kScale = 0.25f;   // codes enter as 4(c + 128)
+    // o = 128 d = 512 k; codes enter as 4(c + 128)
+    static constexpr float kSumScale = -512.f, kScale = 0.25f;
     static constexpr int kDwords = 17;
     typedef PairRaw<kDwords> Raw;
     __device__ static h8 code(const Raw &r, int g, int j)
@@ -308,8 +308,8 @@ struct UQ80 {
 struct UQ40 {
     static constexpr int kBytes = 144, kBlocks = 8, kBlockElems = 32, SB = 32;
     static constexpr bool kOwner = true;
-    static constexpr bool kOwnMin = false;      // o = 8 d = 512 k
-    static constexpr float kSumScale = -512.f, kScale = 0.015625f;   // codes enter as 64c
+    // o = 8 d = 512 k; codes enter as 64c
+    static constexpr float kSumScale = -512.f, kScale = 0.015625f;
     static constexpr int kDwords = 9;
     typedef PairRaw<kDwords> Raw;
     __device__ static h8 code(const Raw &r, int g, int j)
