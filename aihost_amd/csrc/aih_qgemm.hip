@@ -17,7 +17,7 @@
 // of 256 elements: producer waves dequantize W for the next super-step
 // into LDS while four consumer waves multiply the current one, their A
 // fragments loaded straight from the tiled X (see qgemm_kernel).  Large grids
-// use 256 x 64 or 512 x 64 tiles with every wave in both roles
+// use 256 x 64, 512 x 64 or 512 x 128 tiles with every wave in both roles
 // (qgemm256_kernel); products whose grid leaves CUs idle split K over
 // workgroups and sum the partials in a second pass (plan_gemm,
 // launch_split_sum).  The epilogue stores Y or adds into it (the residual add

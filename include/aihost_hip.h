@@ -259,7 +259,9 @@ int aih_qmatvec_fused(aih_ctx *ctx, int type, const void *W, int64_t N, int64_t 
  * count), not on the call; where that workspace cannot grow (during a
  * capture, out of memory), the call fails like the X workspace's.  One of at
  * most 256 rows does so too, in every entry point and with every epilogue
- * alike, with partial sums that fit a workspace set aside by aih_init.
+ * alike, with partial sums that fit the 17 MiB set aside by aih_init.  The
+ * number of splits depends on M: a row's last bits can differ between products
+ * of different row counts (a prompt taken whole or in pieces).
  * Replaces TempF32 + ComputeOps.MatMulWeights for M > 8. */
 int aih_qgemm(aih_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
               const float *X, int64_t M, float *Y);
@@ -346,8 +348,10 @@ int64_t aih_operand_bytes(int64_t M, int64_t K);
  * being captured into a HIP graph, tight serving loops, harnesses that forbid
  * hipMalloc.  Same arguments, routing, kernels and results as
  * aih_matmul_weights_q; the staging memory those kernels need (the partial
- * sums of the 3..8-column matvec, the GEMM's fp16 copy of X: mpad * (2K + 4)
- * bytes, mpad = M rounded up to 32) comes from one static device buffer of
+ * sums of the 3..8-column matvec; the GEMM's fp16 copy of X, mpad * (2K + 4)
+ * bytes with mpad = M rounded up to 32, and behind it the partial sums of a
+ * product of at most 256 rows split over K, which never need more than what is
+ * left) comes from one static device buffer of
  * AIH_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends, instead of
  * the context workspace.  A call that needs more returns AIH_E_SCRATCH
  * before launching anything (at K = 4096 the GEMM takes M up to 2048; at
@@ -439,9 +443,11 @@ int64_t aih_attention_scratch_floats(int32_t n_heads, int32_t max_len);
  * `scratch` (aih_attention_scratch_floats floats); more rows use a tiled
  * kernel with an online softmax on the fp16 matrix cores, each fp32 operand
  * split into two fp16 halves (22 significant bits, products exact, sums in
- * fp32; normwise error about 1e-7), one workgroup per 64-query tile whose
- * two halves take the first and last halves of a long key range and merge
- * in LDS (no workspace).  Calls sharing a scratch must not overlap.
+ * fp32; normwise error about 1e-7), one workgroup per 64-query tile of one
+ * head, whose two halves take the first and last halves of a long key range,
+ * or of two heads (aih_attention_heads_per_workgroup), whose halves share every
+ * key tile; they merge in LDS (no workspace).  Calls sharing a scratch must not
+ * overlap.
  * Replaces ComputeOps.MultiHeadAttention and FusedMHAGenerate
  * (ComputeOps.cs:1015-1102, shaders ComputeShaders.cs:656-733), without the
  * latter's 4096-key limit. */
