@@ -192,21 +192,26 @@ struct DQ40 {
     }
 };
 
-// Bound by HBM.  The loads of a thread's F::kTiles tiles are in flight
-// together, and the stores are non-temporal (the output does not displace the
-// packed weights from the caches).  On MI355X, 32000 x 4096 over rotating
-// tensors, against one tile per grid-stride step with plain stores: Q4_K 225 ->
-// 81 us (7.3 TB/s), Q6_K 128 -> 114, Q8_0 165 -> 107, Q4_0 154 -> 84; 4096 x
-// 4096 Q4_K 19.5 -> 11.9.  Two and four tiles differ by 0-4%, but for Q6_K
-// (122 against 114); eight 95-120; two or four with plain stores 111-114.
+template <bool STREAM>
+__device__ __forceinline__ void store4(f4 v, f4 *to)
+{
+    if (STREAM) __builtin_nontemporal_store(v, to);
+    else *to = v;
+}
+
+// Bound by HBM.  The loads of a thread's kTiles tiles are in flight together.
+// On MI355X, 32000 x 4096 over rotating tensors, against one tile per
+// grid-stride step with plain stores: Q4_K 225 -> 81 us (7.3 TB/s), Q6_K 128 ->
+// 114, Q8_0 165 -> 107, Q4_0 154 -> 84.  Two and four tiles differ by 0-4%, but
+// for Q6_K (122 against 114); Q4_K with eight 95-120, with plain stores 111-114.
+// STREAM: non-temporal stores (launch_type).
 // Step g writes the 4 KB * kTiles of outputs from element 1024 * kTiles * g:
 // thread t's outputs 4 t .. 4 t + 3 of each of the kTiles tiles.
-template <class F, int MODE>
+template <class F, int MODE, int kTiles, bool STREAM>
 __global__ void __launch_bounds__(256)
 dequant_kernel(const uint8_t *__restrict__ q, f4 *__restrict__ out, uint64_t n_blocks)
 {
     constexpr int LPB = F::QK / 4;  // lanes per block
-    constexpr int kTiles = F::kTiles;
     constexpr int step = 256 / LPB * F::BB;   // packed bytes of a tile
     const uint64_t total = n_blocks * LPB;
     const uint64_t groups = (total + 256 * kTiles - 1) / (256 * kTiles);
@@ -219,13 +224,13 @@ dequant_kernel(const uint8_t *__restrict__ q, f4 *__restrict__ out, uint64_t n_b
 #pragma unroll
             for (int u = 0; u < kTiles; ++u) F::load(b + u * step, lane, r[u]);
 #pragma unroll
-            for (int u = 0; u < kTiles; ++u) __builtin_nontemporal_store(F::template value<MODE>(r[u], lane), out + t0 + 256 * u);
+            for (int u = 0; u < kTiles; ++u) store4<STREAM>(F::template value<MODE>(r[u], lane), out + t0 + 256 * u);
         } else {
 #pragma unroll
             for (int u = 0; u < kTiles; ++u)
                 if (t0 + 256 * u < total) {
                     F::load(b + u * step, lane, r[u]);
-                    __builtin_nontemporal_store(F::template value<MODE>(r[u], lane), out + t0 + 256 * u);
+                    store4<STREAM>(F::template value<MODE>(r[u], lane), out + t0 + 256 * u);
                 }
         }
     }
@@ -274,18 +279,40 @@ int launch_embed(aih_ctx *ctx, const void *table, int64_t vocab, int64_t dim, co
     return aih_launch_status();
 }
 
-template <class F>
-int launch_type(aih_ctx *ctx, const void *q, float *out, uint64_t n_blocks, int mode)
+template <class F, int KT, bool STREAM>
+int launch_tiles(aih_ctx *ctx, const void *q, float *out, uint64_t n_blocks, int mode)
 {
-    const uint64_t groups = (n_blocks * (F::QK / 4) + 256 * F::kTiles - 1) / (256 * F::kTiles);
+    const uint64_t groups = (n_blocks * (F::QK / 4) + 256 * KT - 1) / (256 * KT);
     const unsigned grid = (unsigned)std::min<uint64_t>(groups, 1u << 22);
     const uint8_t *qb = static_cast<const uint8_t *>(q);
     f4 *o = reinterpret_cast<f4 *>(out);
     if (mode == AIH_F16_REFCPU)
-        hipLaunchKernelGGL((dequant_kernel<F, AIH_F16_REFCPU>), dim3(grid), dim3(256), 0, ctx->stream, qb, o, n_blocks);
+        hipLaunchKernelGGL((dequant_kernel<F, AIH_F16_REFCPU, KT, STREAM>), dim3(grid), dim3(256), 0, ctx->stream, qb, o,
+                           n_blocks);
     else
-        hipLaunchKernelGGL((dequant_kernel<F, AIH_F16_IEEE>), dim3(grid), dim3(256), 0, ctx->stream, qb, o, n_blocks);
+        hipLaunchKernelGGL((dequant_kernel<F, AIH_F16_IEEE, KT, STREAM>), dim3(grid), dim3(256), 0, ctx->stream, qb, o,
+                           n_blocks);
     return aih_launch_status();
+}
+
+// An output is there to be read: one that the 256 MB memory-side cache can hold
+// is stored plainly, so that its reader finds it there.  Larger ones gain from
+// non-temporal stores.  us for the call alone, and for it and an aih_add that
+// reads all of the output, at K = 4096, plain against non-temporal:
+//   Q6_K   8 MB  3.6, 9.9   against 3.7, 11.2      Q8_0  16 MB  5.0, 16.0 against 4.1, 18.7
+//   Q4_K  67 MB 13.1, 37.1  against 11.6, 41.1     Q6_K  67 MB 13.4, 36.8 against 12.9, 40.8
+//   Q6_K 134 MB 25.3, 69.7  against 24.3, 79.7     Q6_K 197 MB 39.8, 124 against 34.8, 121
+// Fewer than five workgroups per CU at F::kTiles tiles each: one tile per thread
+// (Q6_K 8 MB and its reader 9.9 us against 10.7 with four).
+constexpr uint64_t kStreamBytes = 160u << 20;
+
+template <class F>
+int launch_type(aih_ctx *ctx, const void *q, float *out, uint64_t n_blocks, int mode)
+{
+    const uint64_t bytes = n_blocks * F::QK * sizeof(float), cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    if (bytes > kStreamBytes) return launch_tiles<F, F::kTiles, true>(ctx, q, out, n_blocks, mode);
+    if (bytes >= 5 * cus * (4096 * F::kTiles)) return launch_tiles<F, F::kTiles, false>(ctx, q, out, n_blocks, mode);
+    return launch_tiles<F, 1, false>(ctx, q, out, n_blocks, mode);
 }
 
 }  // namespace

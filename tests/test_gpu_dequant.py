@@ -57,9 +57,24 @@ def test_crafted_blocks_bit_exact(device, orc, qtype, mode):
 @pytest.mark.parametrize("elems", [256, 1792, 2048, 2304, 4096, 6400, 8448])
 @pytest.mark.parametrize("qtype", TYPES)
 def test_workgroup_edges_bit_exact(device, orc, qtype, elems):
-    # a workgroup step covers 2048 outputs (Q6_K 4096): less than one, whole ones, a rest
+    # one tile of 1024 outputs per workgroup step: less than one, whole ones, a rest
     data = crafted_blocks(qtype, elems // QK[qtype], seed=elems + qtype)
     for n in {elems, elems - QK[qtype]} - {0}:
+        part = data[:n // QK[qtype] * BB[qtype]]
+        compare(dequant(device, qtype, part, n, nat.F16_IEEE), orc.dequantize(qtype, part, n, nat.F16_IEEE))
+
+
+# Outputs of 10 MB (Q6_K 20 MB) and more take two (four) tiles per step, and of
+# more than 160 MB non-temporal stores: the first such size on a 256-CU device
+# with whole steps, one block less and a rest in the second tile.
+@pytest.mark.parametrize("first", [1280 * 1024, (160 << 18) + 4096])
+@pytest.mark.parametrize("qtype", TYPES)
+def test_steps_of_several_tiles_bit_exact(device, orc, qtype, first):
+    tiles = 4 if qtype == nat.Q6_K else 2
+    n0 = first * tiles if first < 1 << 22 else first
+    block = crafted_blocks(qtype, 4093, seed=qtype)
+    data = np.resize(block, (n0 + 1280) // QK[qtype] * BB[qtype])
+    for n in ((n0, n0 - QK[qtype], n0 + 1280) if first < 1 << 22 else (n0 + 1280,)):
         part = data[:n // QK[qtype] * BB[qtype]]
         compare(dequant(device, qtype, part, n, nat.F16_IEEE), orc.dequantize(qtype, part, n, nat.F16_IEEE))
 
