@@ -248,25 +248,21 @@ struct UQ6K {
 // 25.9.  Runs of four blocks shared by two lanes in one 8-column tile (half
 // the MFMAs, every byte loaded twice) measured 18.8, 161 and 29.6 us at the
 // 8-column sizes.
-// In a last, partial unit (nb blocks inside the row) single dwords are read,
-// so that a read past the tile's rows returns zeros on its own, and blocks
-// past the row get scale 0 (their activations are staged as zeros).
+// In a last, partial unit (nb blocks inside the row, an even number: K is a
+// multiple of 64) a lane whose pair lies past the row reads the unit's first
+// pair instead and gives its blocks scale 0 (their activations are staged as
+// zeros).
 template <int NW>
 struct PairRaw { uint32_t w[NW]; uint32_t nb; };
 
 template <int NW, bool WHOLE>
 __device__ __forceinline__ void load_pair(Rsrc r, uint32_t rowoff, int q, uint32_t so, int nb, PairRaw<NW> &w)
 {
-    const uint32_t at = rowoff + 4 * NW * q;
+    const uint32_t at = rowoff + 4 * NW * (WHOLE || 2 * q < nb ? q : 0);
     w.nb = WHOLE ? 8u : (uint32_t)nb;
-    if constexpr (WHOLE) {
 #pragma unroll
-        for (int i = 0; i < NW / 4; ++i) put4(w.w + 4 * i, bld16(r, at + 16 * i, so));
-        w.w[NW - 1] = bld4(r, at + 4 * (NW - 1), so);
-    } else {
-#pragma unroll
-        for (int i = 0; i < NW; ++i) w.w[i] = bld4(r, at + 4 * i, so);
-    }
+    for (int i = 0; i < NW / 4; ++i) put4(w.w + 4 * i, bld16(r, at + 16 * i, so));
+    w.w[NW - 1] = bld4(r, at + 4 * (NW - 1), so);
 }
 // Dwords i and i + 1 of the codes of block g (at byte 2 of the pair, or at the
 // dword after its middle), and its scale times f.
