@@ -797,21 +797,23 @@ __device__ __forceinline__ f4 split_sum4(const float *__restrict__ p, int S, int
 // The splits of a GEMM split over K: Y = P_0 + P_1 + ... (in that order),
 // added into Y (Y + sum, the order of the accumulate epilogue) when
 // `accumulate`.  Splits are zs floats apart (a multiple of 4, at least MN).
-// Four elements per thread (16-byte accesses of Y when it is 16-byte aligned).
-// MN fits 32 bits: a split product has fewer tiles than the device has CUs.
-template <bool VEC>
+// Four elements per thread (16-byte accesses of Y when it is 16-byte aligned);
+// ROWS4: N >= 4.  MN fits 32 bits: a split product has fewer tiles than the device has CUs.
+template <bool VEC, bool ROWS4>
 __global__ void __launch_bounds__(256)
-split_k_sum_kernel(const float *__restrict__ P, int S, int64_t MN, uint32_t N, int64_t zs,
+split_k_sum_kernel(const float *__restrict__ P, int S, int64_t MN, uint32_t M, uint32_t N, int64_t zs,
                    const int32_t *__restrict__ E, float *__restrict__ Y, int accumulate)
 {
     for (int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x); i < MN; i += 4 * (int64_t)gridDim.x * 256) {
-        const int e = E[(uint32_t)i / N];   // in flight beside the partials
+        // Four elements lie in the row of element i and the next one (N >= 4), or
+        // past the end; their exponents are in flight beside the partials.
+        const uint32_t m = (uint32_t)i / N, in_row = (m + 1) * N - (uint32_t)i;   // elements left in row m
+        const int e0 = E[m], e1 = E[min(m + 1, M - 1)];
         f4 s = split_sum4(P + i, S, zs);
-        if (N % 4 == 0) {
-            s = undo_row_exp4(s, e);
-        } else {   // the four elements may lie in several rows (past the end: the last row's)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) s[j] = ldexpf(s[j], -E[(uint32_t)min<int64_t>(i + j, MN - 1) / N]);
+        for (int j = 0; j < 4; ++j) {
+            if (ROWS4) s[j] = ldexpf(s[j], j < in_row ? -e0 : -e1);
+            else s[j] = ldexpf(s[j], -E[min((uint32_t)i + j, (uint32_t)MN - 1) / N]);
         }
         if (VEC && i + 4 <= MN) {
             f4 *y = reinterpret_cast<f4 *>(Y + i);
@@ -1059,12 +1061,15 @@ int launch_split_sum(aih_ctx *ctx, const float *P, const GemmPlan &p, int64_t M,
     const int64_t groups = ((M * N + 3) / 4 + 255) / 256;
     const dim3 grid((unsigned)std::min<int64_t>(groups, 8 * cus));
     const int add = epi == kEpiAccumulate ? 1 : 0;
-    if (reinterpret_cast<uintptr_t>(Y) % 16 == 0)
-        hipLaunchKernelGGL(split_k_sum_kernel<true>, grid, dim3(256), 0, ctx->stream, P, p.splits, M * N, (uint32_t)N, zs, E,
-                           Y, add);
+    if (N < 4)
+        hipLaunchKernelGGL((split_k_sum_kernel<false, false>), grid, dim3(256), 0, ctx->stream, P, p.splits, M * N,
+                           (uint32_t)M, (uint32_t)N, zs, E, Y, add);
+    else if (reinterpret_cast<uintptr_t>(Y) % 16 == 0)
+        hipLaunchKernelGGL((split_k_sum_kernel<true, true>), grid, dim3(256), 0, ctx->stream, P, p.splits, M * N, (uint32_t)M,
+                           (uint32_t)N, zs, E, Y, add);
     else
-        hipLaunchKernelGGL(split_k_sum_kernel<false>, grid, dim3(256), 0, ctx->stream, P, p.splits, M * N, (uint32_t)N, zs, E,
-                           Y, add);
+        hipLaunchKernelGGL((split_k_sum_kernel<false, true>), grid, dim3(256), 0, ctx->stream, P, p.splits, M * N, (uint32_t)M,
+                           (uint32_t)N, zs, E, Y, add);
     return aih_launch_status();
 }
 
