@@ -1245,7 +1245,7 @@ struct KVTile {
         const int64_t base = j0 * kv_stride + kvh * kHD;
         const Rsrc rk = make_rsrc(uniform_ptr(Kc + base), bytes), rv = make_rsrc(uniform_ptr(Vc + base), bytes);
         const int kt_key = tid >> 4, kt_ch = tid & 15;
-        const int vt_t = tid / (TH / 2), vt_g = tid / (TH / 8) & 3, vt_d = tid % (TH / 8);
+        const int vt_t = (uint32_t)tid / (TH / 2), vt_g = (uint32_t)tid / (TH / 8) & 3, vt_d = (uint32_t)tid % (TH / 8);
 #pragma unroll
         for (int i = 0; i < KN; ++i) {
             const uint32_t at = (uint32_t)(kt_key + TH / 16 * i) * row + 32 * kt_ch;
@@ -1294,7 +1294,7 @@ struct KVTile {
     __device__ __forceinline__ void split_to_lds(int ek, int ev, int tid, _Float16 *lds) const
     {
         const int kt_key = tid >> 4, kt_ch = tid & 15;
-        const int vt_t = tid / (TH / 2), vt_g = tid / (TH / 8) & 3, vt_d = tid % (TH / 8);
+        const int vt_t = (uint32_t)tid / (TH / 2), vt_g = (uint32_t)tid / (TH / 8) & 3, vt_d = (uint32_t)tid % (TH / 8);
 #pragma unroll
         for (int i = 0; i < KN; ++i) {
             h8 hi, lo;
@@ -1553,17 +1553,19 @@ attn_prefill_kernel(const float *__restrict__ Q, int64_t ldq, const float *__res
 }
 
 // The same products for two heads of one KV head at once, where that still
-// fills the CUs (prefill_pairs).  attn_prefill_kernel is bound by the splitting
-// of K and V into fp16 pairs (352 of 586 VALU instructions per wave and tile)
-// and by its LDS reads (64 KB per wave and tile for 96 MFMAs).  Here a
-// workgroup's eight waves share one image of a 64-key tile (each thread splits
+// fills the CUs (prefill_pairs).  attn_prefill_kernel is bound by its VALU
+// instructions (586 per wave and tile beside 96 MFMAs, 352 of them the splitting
+// of K and V into fp16 pairs) and by its LDS reads (64 KB per wave and tile):
+// counters at 2048 queries, 32 heads over 8, of 184 us a call: VALU issue 75,
+// MFMAs 42, LDS 97, half of that bank conflicts.  Here, of 139 us: VALU 66, MFMAs
+// 42, LDS 46.  A workgroup's eight waves share one image of a 64-key tile (each thread splits
 // half as much, and holds half as many rows in flight), and every K and V
 // fragment feeds the queries of both heads.  Wave w of half h owns the queries
 // 16w .. 16w + 15 of each head and the keys 32h .. 32h + 31 of every tile (score
 // blocks 2h, 2h + 1, product step t = h); the halves merge at the end as above.
 // Two images in LDS, one barrier per tile.
-// On MI355X, 32 heads over 8: 2048 queries 188 -> 142 us, 1024 at
-// position 2000 215 -> 179, 2048 at 2000 492 -> 363; 3.45 us a tile and
+// On MI355X, 32 heads over 8: 2048 queries 184 -> 139 us, 1024 at
+// position 2000 206 -> 177, 2048 at 2000 484 -> 361; 3.45 us a tile and
 // workgroup against 2.45 for one head.  The same form with one head (NB = 1) is
 // 3-5% slower than attn_prefill_kernel, which therefore stays for it.
 __global__ void __launch_bounds__(512, 1)
@@ -2253,10 +2255,11 @@ int aih_add(aih_ctx *ctx, const float *A, const float *B, float *Y, int64_t n)
 // schedule of the query tiles' workgroups over the CUs, in key tiles (the
 // longest workgroup, the mean load, and k + 1 workgroups at least as long as
 // the (k cus + 1)-th on some CU), at the measured 3.45 us a tile for two heads
-// and 2.45 us for one.  A position in device memory counts as 0: the host cannot
-// know it, and one head at a time is never slower than it was.  Measured at
+// and 2.45 us for one.  A position in device memory counts as 0: the host does
+// not know it, and one head at a time is right or the smaller loss.  Measured at
 // 32 heads, one -> two: 512 queries 28.9 -> 40.3 us (128 workgroups on 256
-// CUs), 1024 59 -> 69, 1500 119 -> 94.  Over 91 shapes (4 to 64 heads, 9 to
+// CUs), 1024 59 -> 69, 1500 116 -> 92: the rule takes two from 1345 queries at
+// position 0 and from 513 at 2000.  Over 91 shapes (4 to 64 heads, 9 to
 // 2048 queries, positions 0 to 3000) it picks the faster one, or a tie.
 static bool prefill_pairs(const aih_ctx *ctx, int64_t n_q, int32_t n_heads, int32_t n_kv_heads, int32_t start,
                           int32_t max_len)

@@ -273,16 +273,17 @@ __device__ __forceinline__ void rope_qkv_tile(const f16v &acc0, const f16v &acc1
 //   measured faster there.  Their packed loads run PR super-steps ahead in a
 //   ring of register sets.  A single producer wave per SIMD issues its
 //   dependent conversions at 5 to 7 cycles each; two fill each other's gaps
-//   (4096 x 4096 x 512 per call, four against eight producers: Q4_K 35.1 ->
-//   33.0 us, Q4_0 33.4 -> 32.3, Q6_K 39.5 -> 38.4; 4096 x 14336 x 33 unsplit,
-//   Q4_K 69.3 -> 59.4).  Q8_0, bound by its 34-byte blocks' unaligned loads,
+//   (4096 x 4096 x 512 per call, four against eight producers: 3% in all three
+//   formats, Q4_K 32.8 -> 31.8 us; 4096 x 14336 x 33 unsplit, Q4_K 69.3 ->
+//   59.4).  Twelve waves leave 168 registers a lane: the wave index is held in a
+//   scalar register, or a few would be kept in private memory.  Q8_0, bound by its 34-byte blocks' unaligned loads,
 //   gained nothing there and lost 1-3% where its weights fill the memory
 //   (32000 x 14336 x 64: 198 against 203 us): it keeps four.
 //   Consumers (waves 0..3): wave w owns rows 32w .. 32w+31 of the M tile and
 //   all 64 columns (two 32x32 accumulators sharing each A fragment).  A
 //   fragments come straight from the tiled fp16 copy of X, one super-step
 //   ahead; B fragments from LDS.
-// On MI355X the 4096 x 4096 x 512 Q4_K product takes 33 us per call (the
+// On MI355X the 4096 x 4096 x 512 Q4_K product takes 32-35 us per call (the
 // kernel about 25 us, the X conversion 7.5 us).
 constexpr int SK = 256;            // k per super-step (one barrier)
 constexpr int SC = SK / 64;        // 64-k steps per super-step
@@ -501,11 +502,13 @@ qgemm_kernel(const uint8_t *W, int64_t N, int64_t K, int64_t row_bytes,
 // 256-row workgroup takes about 1.25 times as long as a 128-row one, for
 // twice the outputs.
 // With 64 columns every A fragment is loaded for two MFMAs, 64 bytes per clock
-// and CU through the vector L1 at the full MFMA rate, which is all it gives:
-// the 512 x 64 tile reaches half that rate.  The 512 x 128 tile (NB = 2) halves
-// those loads; its 128 accumulator registers leave room for A one 64-k chunk
-// and B one 16-k slice ahead.  Per call, Q4_K K = 4096: 14336 x 2048 291 -> 237
-// us, 28672 x 512 138 -> 121 us.  Left out one at a time (a copy, 237 us): the
+// and CU through the vector L1 at the full MFMA rate, which is all it gives.
+// Counters of the 512 x 64 tile (14336 x 4096 x 512, its 224 CUs): 28 bytes per
+// clock, the L1's return path busy 74% of the time, the MFMAs 42%.  The 512 x 128
+// tile (NB = 2) halves those loads (x 2048: return path 70%, MFMAs 54% of all
+// CUs, where the 256 x 64 tile has 80% and 43%); its 128 accumulator registers
+// leave room for A one 64-k chunk and B one 16-k slice ahead.  Per call, Q4_K K =
+// 4096: 14336 x 2048 301 -> 245 us, 28672 x 512 145 -> 123 us.  Left out one at a time (a copy, 237 us): the
 // A loads -26 us, the dequantization -36 us, both -55 us: what remains is the
 // MFMAs, and the last round of workgroups.
 constexpr int BM2 = 256;
@@ -963,7 +966,10 @@ struct GemmPlan {
 // it again; a workgroup of them takes about 1.25 and 2.35 times as long as
 // one of 128 rows, one of 512 x 128 about 3.6 times (measured on MI355X;
 // chip full, all four formats: 112-127 us a round of 4096 of K, against 68-76
-// of 512 x 64; nearly empty 82 against 62).  The shape with the fewest such
+// of 512 x 64, that is 3.5 to 4.4 of the 2.35; nearly empty 82 against 62, 3.1:
+// 3.6 is the one constant under which no measured shape lost).  The units were
+// fitted with four producer waves; eight made the 128-row workgroup 3% shorter,
+// which moves no choice by more than a tie.  The shape with the fewest such
 // rounds of workgroups over the device's CUs wins (ties to the smaller tile).
 // Costs in units of 1/20 of a 128-row workgroup.  Products of more than 256
 // rows whose 512-row tiles leave CUs idle split K over workgroups: S splits
@@ -979,9 +985,9 @@ struct GemmPlan {
 // its traffic at 2.5 TB/s.  Every entry point and epilogue splits a shape
 // alike, so the operand image and the partial sums together stay within the
 // allocation-free entry point's buffer.
-// Measured per call (Q4_K / Q6_K, whole -> split): 4096 x 14336 x 33 69 -> 28
-// / 82 -> 32 us, 4096 x 4096 x 33 24 -> 15 / 28 -> 17, x 256 27 -> 24 / 31 ->
-// 26, 1024 x 14336 x 64 71 -> 21 / 84 -> 23, 8192 x 4096 x 9 25 -> 18 / 30 ->
+// Measured per call (Q4_K / Q6_K, whole -> split): 4096 x 14336 x 33 70 -> 26
+// / 83 -> 31 us, 4096 x 4096 x 33 23 -> 14 / 28 -> 16, x 256 26 -> 22 / 31 ->
+// 25, 1024 x 14336 x 64 69 -> 19 / 82 -> 23, 8192 x 4096 x 9 24 -> 17 / 29 ->
 // 21; over 216 sizes of N 1024-32000, K 1024-14336 and M 9-256 none slower
 // than the runs differ.
 int64_t split_stride(int64_t M, int64_t N) { return (M * N + 3) / 4 * 4; }

@@ -243,11 +243,13 @@ struct UQ6K {
 // two blocks are one scaling group (64 elements), so that large activations
 // elsewhere in the unit cost them no bits of their hi/lo pairs.
 // On MI355X per call (pieces of 8 bytes -> owned pairs of blocks): Q4_0 14336 x
-// 4096 4 columns 32.9 -> 13.5 us, 8 columns 32.1 -> 18.2, 32000 x 14336 x 8
-// 262 -> 129; Q8_0 14336 x 4096 x 4 30.8 -> 16.5, 4096 x 14336 x 8 35.7 ->
-// 25.9.  Runs of four blocks shared by two lanes in one 8-column tile (half
-// the MFMAs, every byte loaded twice) measured 18.8, 161 and 29.6 us at the
-// 8-column sizes.
+// 4096 4 columns 32.6 -> 13.1 us, 8 columns 31.5 -> 17.1 (the address unit busy
+// 58k -> 17k cycles a CU), 32000 x 14336 x 8 252 -> 106; Q8_0 14336 x 4096 x 4
+// 30.3 -> 15.8, 4096 x 14336 x 8 35.0 -> 20.6.  One unit at 8 columns, with its
+// twice as many MFMAs, takes 0.2-0.4 us more (2048 x 64: 3.4 -> 3.9).  Runs of four
+// blocks shared by two lanes in one 8-column tile (half the MFMAs, every byte
+// loaded twice) were slower at the 8-column sizes (18.8 us where this form took
+// 18.2, 161 against 129, 29.6 against 25.9).
 // In a last, partial unit (nb blocks inside the row, an even number: K is a
 // multiple of 64) a lane whose pair lies past the row reads the unit's first
 // pair instead and gives its blocks scale 0 (their activations are staged as
