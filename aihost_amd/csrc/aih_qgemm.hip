@@ -966,12 +966,13 @@ struct GemmPlan {
 // it again; a workgroup of them takes about 1.25 and 2.35 times as long as
 // one of 128 rows, one of 512 x 128 about 3.6 times (measured on MI355X;
 // chip full, all four formats: 112-127 us a round of 4096 of K, against 68-76
-// of 512 x 64, that is 3.5 to 4.4 of the 2.35; nearly empty 82 against 62, 3.1:
-// 3.6 is the one constant under which no measured shape lost).  The units were
-// fitted with four producer waves; eight made the 128-row workgroup 3% shorter,
-// which moves no choice by more than a tie.  The shape with the fewest such
-// rounds of workgroups over the device's CUs wins (ties to the smaller tile).
-// Costs in units of 1/20 of a 128-row workgroup.  Products of more than 256
+// of 512 x 64; nearly empty 82 against 62: 3.6 lies between).  The units were
+// fitted with four producer waves.  With eight, every tile forced in turn over
+// 64 unsplit products (all formats, 257 to 2048 rows, N 1096 to 31832, K 1024 to
+// 7936): the plan's is the fastest or within 2%, but for three Q4_0 products
+// where 128 rows would be 6 to 10% faster than its 512 x 64.  The shape with
+// the fewest such rounds of workgroups over the device's CUs wins (ties to the
+// smaller tile).  Costs in units of 1/20 of a 128-row workgroup.  Products of more than 256
 // rows whose 512-row tiles leave CUs idle split K over workgroups: S splits
 // of at least two whole super-steps, partial sums in the second workspace,
 // then a summing pass (estimated at 5 TB/s over the partials, Y and the
